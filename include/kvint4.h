@@ -255,9 +255,16 @@ int kvq_decode_step_noalloc(const void* q, int q_dtype, const int64_t* q_strides
  * the device, the key range is split and the splits' partials are merged in
  * a second launch through it; NULL (or too small) runs unsplit. Calls that
  * overlap in time must not share a workspace.
+ * With at least kvq_prefill_attn_staged_workspace_bytes(...) bytes (16-byte
+ * aligned; never less than the other figure, at most 256 MiB of images plus
+ * the split's partials) long blocks dequantize K and V once into it, in
+ * matrix-operand order, instead of once per row block: the same rounding, in
+ * two launches per group of (batch, KV head) units, and the faster route.
  */
 int64_t kvq_prefill_attn_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t D,
                                          int64_t Sk);
+int64_t kvq_prefill_attn_staged_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t D,
+                                                int64_t Sk);
 int kvq_prefill_attn(const void* q, int q_dtype, const int64_t* q_strides,
                      const void* k_packed, const int64_t* kp_strides,
                      const void* k_scales, const int64_t* ks_strides,

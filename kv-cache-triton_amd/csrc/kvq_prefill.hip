@@ -81,6 +81,11 @@ struct PrefillArgs {
   int n_split;
   float* ws_o;   // [unit][split][rows][D]
   float* ws_ml;  // [unit][split][rows][2]
+  // staged route: operand images of the units u0 .. u0 + n_units - 1 (unit =
+  // b * Hkv + kvh), `tiles` tiles of 16 D pieces of 16 bytes each
+  uint4* img;
+  int u0, n_units, tiles;
+  int q_vec, o_vec, kv_vec;  // 16-byte query rows, 8-byte output pieces, 16-byte K / 4-byte V code loads
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t prefill_rsrc(const void* p, uint32_t bytes) {
@@ -112,6 +117,24 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 template <bool S_F16>
 __device__ __forceinline__ float scale_f32(uint32_t bits) {
   return S_F16 ? f16_bits_to_f32(bits & 0xffffu) : bf16_bits_to_f32(bits & 0xffffu);
+}
+
+// Eight elements of a query row, as one 16-byte load where every row is
+// aligned for it (vec), else element by element.
+__device__ __forceinline__ uint4 load8(const uint16_t* p, bool vec) {
+  if (vec) return *(const uint4*)p;
+  return make_uint4((uint32_t)p[0] | ((uint32_t)p[1] << 16), (uint32_t)p[2] | ((uint32_t)p[3] << 16),
+                    (uint32_t)p[4] | ((uint32_t)p[5] << 16), (uint32_t)p[6] | ((uint32_t)p[7] << 16));
+}
+
+// Four output elements, as one 8-byte store where every row is aligned for it.
+__device__ __forceinline__ void store4(uint16_t* p, uint32_t w0, uint32_t w1, bool vec) {
+  if (vec) {
+    *(uint2*)p = make_uint2(w0, w1);
+    return;
+  }
+  p[0] = (uint16_t)w0; p[1] = (uint16_t)(w0 >> 16);
+  p[2] = (uint16_t)w1; p[3] = (uint16_t)(w1 >> 16);
 }
 
 // The tile's share of one thread dequantized as (n - 8) sc directly (the
@@ -148,13 +171,11 @@ __device__ __attribute__((noinline)) void store_tile_direct(uint16_t* k_dst, uin
 // RB = 16-row blocks per wave (1 or 2): with two, every K and V fragment read
 // from LDS feeds two MFMAs, halving LDS traffic and dequantize work per row.
 // Two row blocks per wave must stay within 256 registers (two waves per
-// SIMD): one more register halves the occupancy. NW = waves per workgroup
-// (4, or 8 for D = 128 with two row blocks): the workgroup's threads share
-// the dequantize of each K/V tile, so eight waves (one workgroup per CU
-// instead of two of four) halve its VALU per wave.
-template <int D, bool F16, bool S_F16, int RB, bool PAGED, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(RB == 2 ? 2 : 1)))
+// SIMD): one more register halves the occupancy.
+template <int D, bool F16, bool S_F16, int RB, bool PAGED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RB == 2 ? 2 : 1)))
 void prefill_attn_kernel(const PrefillArgs a) {
+  constexpr int NW = 4;  // waves per workgroup
   constexpr int NT = 64 * NW;
   constexpr int ROWS = kWaveRows * NW * RB;  // query rows per workgroup
   constexpr int KP = D + 8;      // K tile row pitch in LDS (elements)
@@ -229,12 +250,9 @@ void prefill_attn_kernel(const PrefillArgs a) {
         a.q + (int64_t)b * a.qs_b + (int64_t)head[r] * a.qs_h + (int64_t)(row_ok[r] ? s[r] : 0) * a.qs_s;
 #pragma unroll
     for (int kk = 0; kk < NK; ++kk) {
-      const uint16_t* p = qr + 32 * kk + 8 * lg;
-      uint32_t x[4];
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-        x[w] = row_ok[r] ? ((uint32_t)p[2 * w] | ((uint32_t)p[2 * w + 1] << 16)) ^ qneg : 0u;
-      qf[r][kk] = make_uint4(x[0], x[1], x[2], x[3]);
+      const uint32_t keep = row_ok[r] ? 0xffffffffu : 0u;
+      const uint4 x = load8(qr + 32 * kk + 8 * lg, a.q_vec);
+      qf[r][kk] = make_uint4((x.x ^ qneg) & keep, (x.y ^ qneg) & keep, (x.z ^ qneg) & keep, (x.w ^ qneg) & keep);
     }
   }
 
@@ -492,7 +510,7 @@ void prefill_attn_kernel(const PrefillArgs a) {
     l_tot += __shfl_xor(l_tot, 32);
     if (a.n_split > 1) {  // partial of this split, merged by prefill_merge_kernel
       const int rr = wave * kWaveRows * RB + 16 * r + lq;
-      const int64_t slot = ((((int64_t)b * a.row_blocks + blk) * a.Hkv + kvh) * a.n_split + sp) * ROWS + rr;
+      const int64_t slot = (((int64_t)blk * a.n_units + b * a.Hkv + kvh) * a.n_split + sp) * ROWS + rr;
       float* po = a.ws_o + slot * D;
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
@@ -507,100 +525,562 @@ void prefill_attn_kernel(const PrefillArgs a) {
       for (int nb = 0; nb < NB; ++nb) {
         const uint32_t w0 = pack2<F16>(o[r][nb][0] * inv, o[r][nb][1] * inv);
         const uint32_t w1 = pack2<F16>(o[r][nb][2] * inv, o[r][nb][3] * inv);
-        uint16_t* p = orow + 16 * nb + 4 * lg;
-        p[0] = (uint16_t)w0; p[1] = (uint16_t)(w0 >> 16);
-        p[2] = (uint16_t)w1; p[3] = (uint16_t)(w1 >> 16);
+        store4(orow + 16 * nb + 4 * lg, w0, w1, a.o_vec);
       }
     }
   }
 }
 
-// Combines the n_split partials of one query row (log-sum-exp in base 2):
-// one workgroup of D threads per (unit, row), thread d owns output dim d.
+// ---------------------------------------------------------------------------
+// Staged route, for long query blocks. The kernel above dequantizes every K/V
+// tile again in every row block (a 16K prompt at GQA 4: 256 times), and its
+// VALU work (356 instructions per tile and wave against 64 matrix
+// instructions, of which about 90 dequantize and most of the rest move the
+// 16x16 score blocks) is what bounds it. Here stage_kv_kernel dequantizes
+// each tile once, into workspace, in the order the matrix operands are read
+// (an "image": D * 256 bytes per 64-key tile), and prefill_staged_kernel
+// copies images to LDS with direct loads and spends its VALU on the softmax
+// alone.
+//
+// Operands of v_mfma_f32_32x32x16 (lane l: i = l % 32, g = l / 32): A[i][k]
+// and B[k][n] at lane (i or n, k / 8), register k % 8; C[r][n] at lane n +
+// 32 ((r / 4) % 2), register 4 (r / 8) + r % 4. With S^T = K Q^T a lane then
+// holds, of query row n, keys 32 kb + 8 (r / 4) + 4 g + r % 4 (register r of
+// block kb); registers 8 h .. 8 h + 7 are the eight keys {4 g .. 4 g + 3, 8 +
+// 4 g .. 8 + 4 g + 3} of 16-key step t = 2 kb + h, and are the lane's B
+// operand of O^T += V^T P^T for that step if V^T's k order is the same. The
+// images hold
+//   K: [kb][kk][lane] 16-byte pieces, key 32 kb + i, dims 16 kk + 8 g .. + 7
+//   V: [db][t][lane] 16-byte pieces, dim 32 db + i, the eight keys above
+// so that every operand read is one conflict-free 16-byte LDS read at lane *
+// 16, and an image moves to LDS as it is.
+
+// 16 code bytes at p (any alignment unless vec)
+__device__ __forceinline__ uint4 load16(const uint8_t* p, bool vec) {
+  if (vec) return *(const uint4*)p;
+  uint32_t w[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    w[j] = (uint32_t)p[4 * j] | ((uint32_t)p[4 * j + 1] << 8) | ((uint32_t)p[4 * j + 2] << 16) |
+           ((uint32_t)p[4 * j + 3] << 24);
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+__device__ __forceinline__ uint32_t load4(const uint8_t* p, bool vec) {
+  if (vec) return *(const uint32_t*)p;
+  return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
+}
+
+// Cache row of token t of sequence b, or -1 (past Sk, or no block holds it).
+__device__ __forceinline__ int64_t stage_row(const PrefillArgs& a, int b, int t) {
+  if (t >= a.Sk) return -1;
+  if (!a.bt) return t;
+  const int pg = t >> a.page_shift;
+  if (pg >= a.bt_cols) return -1;
+  const int32_t blk = a.bt[(int64_t)b * a.bt_stride + pg];
+  if (blk < 0 || blk >= a.n_blocks) return -1;
+  return ((int64_t)blk << a.page_shift) | (t & ((1 << a.page_shift) - 1));
+}
+
+// One workgroup dequantizes 256 / D tiles of one unit. K: a thread takes 16
+// code bytes of one key (32 dims, one scale), consecutive threads consecutive
+// keys, so its four stores are pieces of contiguous 512-byte runs. V: a thread
+// takes one code dword (8 dims) of the eight keys of an operand piece and
+// stores the eight dims' pieces, 128 contiguous bytes. Memory-bound, and small
+// beside the attention: 16K keys of 8 heads (18.9 MB in, 67 MB out) once per
+// layer. The numerics are kvq_dequantize's; keys without a row are zeros.
+template <int D, bool F16, bool S_F16>
+__global__ __launch_bounds__(256) void stage_kv_kernel(const PrefillArgs a) {
+  constexpr int TPB = 256 / D;  // tiles per workgroup
+  constexpr int KS = D / 16;    // 16-dim steps
+  constexpr int KIMG = 8 * D;   // pieces of the K part of an image
+  __shared__ __align__(16) uint4 v_img[TPB * KIMG];
+  const int tid = threadIdx.x;
+  const int lu = blockIdx.y, unit = a.u0 + lu;
+  const int b = unit / a.Hkv, kvh = unit % a.Hkv;
+  const int tile0 = blockIdx.x * TPB;
+  uint4* img = a.img + (int64_t)lu * a.tiles * (2 * KIMG);
+  const uint8_t* kp = a.kp + (int64_t)b * a.kps_b + (int64_t)kvh * a.kps_h;
+  const uint16_t* ks = a.ks + (int64_t)b * a.kss_b + (int64_t)kvh * a.kss_h;
+  const uint8_t* vp = a.vp + (int64_t)b * a.vps_b + (int64_t)kvh * a.vps_h;
+  const uint16_t* vs = a.vs + (int64_t)b * a.vss_b + (int64_t)kvh * a.vss_h;
+
+  // every load of the thread first (rows without data read nothing)
+  uint4 kw[2];
+  uint32_t ksc[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const int it = tid + 256 * n;
+    const int key = it % 64, part = (it / 64) % (D / 32), tile = tile0 + it / (2 * D);
+    const int64_t r = stage_row(a, b, tile * 64 + key);
+    kw[n] = make_uint4(0x88888888u, 0x88888888u, 0x88888888u, 0x88888888u);
+    ksc[n] = 0u;
+    if (r >= 0) {
+      kw[n] = load16(kp + r * a.kps_s + 16 * part, a.kv_vec);
+      ksc[n] = ks[r * a.kss_s + (32 * part) / a.G];
+    }
+  }
+  const int vj = tid % (D / 8), vkg = (tid / (D / 8)) % 8, vtile = tile0 + tid / D;
+  uint32_t vw[8], vsc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int t = vtile * 64 + 16 * (vkg >> 1) + 4 * (vkg & 1) + (e & 3) + 8 * (e >> 2);
+    const int64_t r = stage_row(a, b, t);
+    vw[e] = 0x88888888u;
+    vsc[e] = 0u;
+    if (r >= 0) {
+      vw[e] = load4(vp + r * a.vps_s + 4 * vj, a.kv_vec);
+      vsc[e] = vs[r * a.vss_s + (8 * vj) / a.G];
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const int it = tid + 256 * n;
+    const int key = it % 64, part = (it / 64) % (D / 32), tile = tile0 + it / (2 * D);
+    if (tile >= a.tiles) continue;
+    const float sc = scale_f32<S_F16>(ksc[n]);
+    const uint32_t w[4] = {kw[n].x, kw[n].y, kw[n].z, kw[n].w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // dims 32 part + 8 j .. + 7: step 2 part + j / 2, g = j % 2
+      uint32_t pk[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        pk[x] = pack2<F16>((float)((int)((w[j] >> (8 * x)) & 15u) - 8) * sc,
+                           (float)((int)((w[j] >> (8 * x + 4)) & 15u) - 8) * sc);
+      img[(int64_t)tile * (2 * KIMG) + ((key >> 5) * KS + 2 * part + (j >> 1)) * 64 + 32 * (j & 1) + (key & 31)] =
+          make_uint4(pk[0], pk[1], pk[2], pk[3]);
+    }
+  }
+  // V pieces through LDS: a thread's eight pieces are 128 contiguous bytes, so
+  // stored straight to memory each instruction would touch 64 lines in part.
+  // Thread vj takes its dims in the order (x + vj) % 8, which spreads an
+  // instruction's pieces over all banks.
+  {
+    uint4* dst = v_img + (vtile - tile0) * KIMG + ((vj >> 2) * 4 + (vkg >> 1)) * 64 + 32 * (vkg & 1) + 8 * (vj & 3);
+    float sc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sc[e] = scale_f32<S_F16>(vsc[e]);
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      const int d = (x + vj) & 7;
+      uint32_t pk[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        pk[e] = pack2<F16>((float)((int)((vw[2 * e] >> (4 * d)) & 15u) - 8) * sc[2 * e],
+                           (float)((int)((vw[2 * e + 1] >> (4 * d)) & 15u) - 8) * sc[2 * e + 1]);
+      dst[d] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {  // TPB * KIMG = 2048 pieces
+    const int i = tid + 256 * j, tile = tile0 + i / KIMG;
+    if (tile < a.tiles) img[(int64_t)tile * (2 * KIMG) + KIMG + i % KIMG] = v_img[i];
+  }
+}
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+template <bool F16>
+__device__ __forceinline__ f32x16_t mfma3216(uint4 a, uint4 b, f32x16_t c) {
+  if constexpr (F16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// max over the two lanes of a query row (l, l + 32)
+__device__ __forceinline__ float pair_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
+  const uint32_t r0 = r[0], r1 = r[1];
+  return __builtin_elementwise_maximum(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
+}
+__device__ __forceinline__ float pair_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
+  const uint32_t r0 = r[0], r1 = r[1];
+  return __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+}
+
+// 16-byte direct loads, global to LDS: lane l's piece of the wave's 1 KB
+// goes to LDS byte address dst + 16 l (dst wave-uniform). Written as asm,
+// not with the builtin: the compiler waits for every direct load in flight
+// before any LDS read, while these fill a buffer that nobody reads until the
+// workgroup has passed `arrive` below. The load has no destination register;
+// the wait is the s_waitcnt vmcnt(0) there (the compiler's own vmcnt waits can
+// only become longer by loads it does not count). M0 holds the LDS address; the
+// s_nop covers the wait state between writing and using it.
+__device__ __forceinline__ void load_to_lds(const uint4* src, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "memory", "m0");
+}
+
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}
+
+// NW waves of 32 query rows each. Per 64-key tile and wave: 16 + 16 matrix
+// instructions (D = 128) and about 140 VALU. The loop is pipelined by one tile
+// on either side of the softmax, so that the block that exponentiates tile i
+// also holds the S^T products of tile i + 1 and the PV products of tile i - 1,
+// all independent of it: a SIMD issues VALU between the 32-cycle matrix
+// instructions of the same wave (a probe: 12 FMAs beside each
+// v_mfma_f32_32x32x16, two waves per SIMD, take the time of the FMAs alone;
+// beside 16x16x32 ones, or in another phase of the wave, most of it is added).
+// K images are two buffers deep ahead of the softmax, V images one behind it:
+// tile i reads K buffer and V buffer (i + 1) % 2 (tiles i + 1 and i - 1) while
+// tiles i + 2 (K) and i (V) are loaded into buffers i % 2.
+// Measured against the kernel above: a 16K prompt (32 query heads, 8 KV heads,
+// D = 128, bf16) 2.38 -> 1.88 ms per layer, 925 -> 1170 TF/s; 777 fp16 queries
+// over 9001 keys 317 -> 142 us with the split chosen in staged_plan and the
+// merge below. At the prompt the matrix cores are busy 62 % of the cycles and
+// the clock falls to about 1.75 GHz under the load (a large bf16 matrix
+// product reaches 1370 TF/s on the same card); four waves per workgroup
+// measured 3 % slower there, a barrier every second tile (128 KB of LDS) 3 %.
+template <int D, bool F16, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void prefill_staged_kernel(const PrefillArgs a) {
+  constexpr int ROWS = 32 * NW;
+  constexpr int KS = D / 16;   // 16-dim steps of S^T
+  constexpr int NDB = D / 32;  // 32-dim blocks of O^T
+  constexpr int KIMG = 8 * D;  // 16-byte pieces of a K (or V) image
+  __shared__ __align__(16) uint4 k_lds[2][KIMG];
+  __shared__ __align__(16) uint4 v_lds[2][KIMG];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 31, lg = lane >> 5;
+  // workgroup -> (unit fastest, so that one head's row blocks share an XCD and
+  // its L2; row blocks with the most keys first)
+  int wg = blockIdx.x;
+  const int lu = wg % a.n_units;
+  wg /= a.n_units;
+  const int sp = wg % a.n_split;
+  const int blk = a.row_blocks - 1 - wg / a.n_split;
+  const int unit = a.u0 + lu;
+  const int b = unit / a.Hkv, kvh = unit % a.Hkv;
+
+  // this lane's query row and the keys it may attend: [0, lim)
+  const int R0 = blk * ROWS + wave * 32, R = R0 + ln;
+  const int s = R / a.ratio, head = kvh * a.ratio + R % a.ratio;
+  const bool row_ok = s < a.Sq;
+  auto clamp_keys = [&](int l) { return l < 0 ? 0 : (l > a.Sk ? a.Sk : l); };
+  const int lim = row_ok ? clamp_keys(a.causal ? a.Sk - a.Sq + s + 1 : a.Sk) : 0;
+  // keys every row of the wave may attend (the first row's; a wave with no row
+  // masks nothing, its rows are never stored), keys any row of the workgroup
+  // attends, and this split's tiles of them
+  const int s0 = R0 / a.ratio;
+  const int lim_wave = s0 < a.Sq ? clamp_keys(a.causal ? a.Sk - a.Sq + s0 + 1 : a.Sk) : 0x7fffffff;
+  const int r_last = min((blk + 1) * ROWS, a.Sq * a.ratio) - 1;
+  const int kend = clamp_keys(a.causal ? a.Sk - a.Sq + r_last / a.ratio + 1 : a.Sk);
+  const int tiles_all = (kend + kKeys - 1) / kKeys;
+  const int tps = (tiles_all + a.n_split - 1) / a.n_split;
+  const int tile_lo = sp * tps;
+  const int n = min(tiles_all, tile_lo + tps) - tile_lo;  // tiles of this workgroup (<= 0: none)
+
+  // queries as the B operand: lane (ln, lg) holds dims 16 kk + 8 lg .. + 7 of
+  // its row (rows past Sq are zero); the sign of sm_scale goes into them and
+  // scores reach the softmax as fma(s, c, -m), c = |sm_scale| log2(e) > 0, as
+  // in prefill_attn_kernel
+  const float c = fmaxf(fabsf(a.scale_log2), 1.0e-30f);
+  const uint32_t qneg = a.scale_log2 < 0.0f ? 0x80008000u : 0u;
+  uint4 qf[KS];
+  {
+    const uint16_t* qr = a.q + (int64_t)b * a.qs_b + (int64_t)head * a.qs_h + (int64_t)(row_ok ? s : 0) * a.qs_s;
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) {
+      const uint4 x = load8(qr + 16 * kk + 8 * lg, a.q_vec);
+      const uint32_t keep = row_ok ? 0xffffffffu : 0u;
+      qf[kk] = make_uint4((x.x ^ qneg) & keep, (x.y ^ qneg) & keep, (x.z ^ qneg) & keep, (x.w ^ qneg) & keep);
+    }
+  }
+
+  f32x16_t o[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) o[db][j] = 0.0f;
+  float m_run = kNegP, l_run = 0.0f;
+
+  const uint4* img = a.img + ((int64_t)lu * a.tiles + tile_lo) * (2 * KIMG);
+  // image part `which` (0 K, 1 V) of local tile i (past the last: the last)
+  auto fetch = [&](int which, int i, const uint4* dst) {
+    const uint4* src = img + (int64_t)min(i, n - 1) * (2 * KIMG) + which * KIMG + lane;
+#pragma unroll
+    for (int j = 0; j < KIMG / 64 / NW; ++j) {
+      const int ch = wave + NW * j;
+      load_to_lds(src + ch * 64, lds_address(dst) + ch * 1024u);
+    }
+  };
+  auto arrive = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's direct loads are in LDS
+    __syncthreads();
+  };
+  auto scores = [&](const uint4* kt, f32x16_t (&st)[2]) {
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const f32x16_t zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        st[kb] = mfma3216<F16>(kt[(kb * KS + kk) * 64 + lane], qf[kk], kk == 0 ? zero : st[kb]);
+      }
+  };
+  auto values = [&](const uint4* vt, const uint4 (&p)[4]) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) o[db] = mfma3216<F16>(vt[(db * 4 + t) * 64 + lane], p[t], o[db]);
+  };
+
+  // tile i of this workgroup: sc = its scores, sn = the next tile's (computed
+  // here), pp = the previous tile's weights, pc = its own (computed here)
+  auto step = [&](f32x16_t (&sc)[2], f32x16_t (&sn)[2], const uint4 (&pp)[4], uint4 (&pc)[4], int i, int par) {
+    fetch(0, i + 2, k_lds[par]);
+    fetch(1, i, v_lds[par]);
+    const int t0 = (tile_lo + i) * kKeys;
+    if (t0 + kKeys > lim_wave) {
+      // only tiles where some row may not attend every key (the causal
+      // diagonal, the last partial tile): scores of excluded keys to -inf
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (t0 + 32 * kb + 8 * (r >> 2) + 4 * lg + (r & 3) >= lim) sc[kb][r] = -__builtin_inff();
+    }
+    float mx = sc[0][0];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = __builtin_elementwise_maximum(mx, sc[kb][r]);
+    const float mt = pair_max(mx) * c;
+    // lazy running max, as in prefill_attn_kernel; the rescale of O waits for
+    // the previous tile's products below, which are in the old reference
+    const bool grow = __builtin_amdgcn_ballot_w64(mt > m_run + kLazyMaxP) != 0;
+    const float m_new = grow ? fmaxf(m_run, mt) : m_run;
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    m_run = m_new;
+    l_run *= alpha;
+    const uint4* kt = k_lds[par ^ 1];
+    const uint4* vt = v_lds[par ^ 1];
+    scores(kt, sn);
+    values(vt, pp);
+    float ls[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      uint32_t w[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int kb = t >> 1, r = 8 * (t & 1) + 2 * x;
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kb][r], c, -m_run));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kb][r + 1], c, -m_run));
+        ls[0] += p0;
+        ls[1] += p1;
+        w[x] = pack2<F16>(p0, p1);
+      }
+      pc[t] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    l_run += ls[0] + ls[1];
+    // one scheduling region: between two matrix instructions an operand read and
+    // a share of the softmax (the row max first, exponentials after it); the
+    // empty asm keeps the results from being sunk into the next tile
+    constexpr int NM = 2 * KS + 4 * NDB;  // matrix instructions of a tile
+    constexpr int VM = 128 / NM;          // VALU between two of them
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int g = 0; g < NM; ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (g < NM / 5) {
+        __builtin_amdgcn_sched_group_barrier(0x002, VM, 0);
+      } else {
+        __builtin_amdgcn_sched_group_barrier(0x400, 32 / NM, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, VM - 1, 0);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(pc[t].x), "+v"(pc[t].y), "+v"(pc[t].z), "+v"(pc[t].w));
+    asm volatile("" : "+v"(sn[0]), "+v"(sn[1]), "+v"(l_run));
+    if (grow) {
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) o[db] *= alpha;
+    }
+    arrive();
+  };
+
+  if (n > 0) {
+    const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
+    fetch(0, 0, k_lds[0]);
+    fetch(0, 1, k_lds[1]);
+    for (int j = tid; j < KIMG; j += 64 * NW) v_lds[1][j] = zero4;  // "tile -1": weights 0 times finite values
+    arrive();
+    f32x16_t sA[2], sB[2];
+    uint4 pA[4], pB[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) pB[t] = zero4;
+    scores(k_lds[0], sA);
+    __syncthreads();  // every wave has read K buffer 0, which tile 0 refills
+    int i = 0;
+    for (; i + 1 < n; i += 2) {
+      step(sA, sB, pB, pA, i, 0);
+      step(sB, sA, pA, pB, i + 1, 1);
+    }
+    if (i < n) {
+      step(sA, sB, pB, pA, i, 0);
+      values(v_lds[0], pA);
+    } else {
+      values(v_lds[1], pB);
+    }
+  }
+
+  // normalise and store: lane (ln, lg) holds dims 32 db + 8 j + 4 lg .. + 3 of
+  // its row in registers 4 j .. 4 j + 3 of block db
+  const float l_tot = pair_sum(l_run);
+  if (a.n_split > 1) {  // partial of this split, merged by prefill_merge_kernel
+    const int64_t slot = (((int64_t)blk * a.n_units + lu) * a.n_split + sp) * ROWS + wave * 32 + ln;
+    float* po = a.ws_o + slot * D;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *(float4*)(po + 32 * db + 8 * j + 4 * lg) =
+            make_float4(o[db][4 * j], o[db][4 * j + 1], o[db][4 * j + 2], o[db][4 * j + 3]);
+    if (lg == 0) *(float2*)(a.ws_ml + 2 * slot) = make_float2(m_run, l_tot);
+    return;
+  }
+  if (!row_ok) return;
+  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+  uint16_t* orow = a.out + (int64_t)b * a.os_b + (int64_t)head * a.os_h + (int64_t)s * a.os_s;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t w0 = pack2<F16>(o[db][4 * j] * inv, o[db][4 * j + 1] * inv);
+      const uint32_t w1 = pack2<F16>(o[db][4 * j + 2] * inv, o[db][4 * j + 3] * inv);
+      store4(orow + 32 * db + 8 * j + 4 * lg, w0, w1, a.o_vec);
+    }
+}
+
+// Combines the n_split partials of the query rows (log-sum-exp in base 2): a
+// thread owns four dims of one row, 256 threads 1024 / D rows of one row
+// block (rows = rows per row block). Memory-bound: it reads every partial
+// once, in 16-byte pieces.
 template <int D, bool F16>
-__global__ __launch_bounds__(D) void prefill_merge_kernel(const PrefillArgs a, int rows) {
-  const int64_t g = blockIdx.x;
-  const int rr = (int)(g % rows);
-  const int64_t unit = g / rows;  // (b * row_blocks + blk) * Hkv + kvh
-  const int kvh = (int)(unit % a.Hkv);
-  const int64_t t = unit / a.Hkv;
-  const int blk = (int)(t % a.row_blocks);
-  const int b = (int)(t / a.row_blocks);
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs a, int rows) {
+  constexpr int RPW = 1024 / D;  // rows per workgroup (divides rows)
+  const int per = rows / RPW;    // workgroups per row block
+  const int rr = (int)(blockIdx.x % per) * RPW + threadIdx.x / (D / 4);
+  const int t = blockIdx.x / per;
+  const int lu = t % a.n_units, blk = t / a.n_units;
+  const int unit = a.u0 + lu;
+  const int b = unit / a.Hkv, kvh = unit % a.Hkv;
   const int R = blk * rows + rr;
   const int s = R / a.ratio;
   if (s >= a.Sq) return;
   const int head = kvh * a.ratio + R % a.ratio;
-  const int d = threadIdx.x;
-  const int64_t slot0 = unit * a.n_split * rows + rr;  // split sp: slot0 + sp * rows
-  float M = kNegP;
-  for (int sp = 0; sp < a.n_split; ++sp) M = fmaxf(M, a.ws_ml[2 * (slot0 + (int64_t)sp * rows)]);
-  float L = 0.0f, acc = 0.0f;
-  for (int sp = 0; sp < a.n_split; ++sp) {
-    const int64_t slot = slot0 + (int64_t)sp * rows;
-    const float2 ml = *(const float2*)(a.ws_ml + 2 * slot);
-    const float w = __builtin_amdgcn_exp2f(ml.x - M);
-    L += ml.y * w;
-    acc += a.ws_o[slot * D + d] * w;
+  const int d = 4 * (threadIdx.x % (D / 4));
+  const int64_t slot0 = (int64_t)t * a.n_split * rows + rr;  // split sp: slot0 + sp * rows
+  // batches of eight splits with all loads in flight together, folded with a
+  // running max (one load at a time, a merge of many splits was a chain of
+  // round trips)
+  float M = kNegP, L = 0.0f;
+  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int s0 = 0; s0 < a.n_split; s0 += 8) {
+    float2 ml[8];
+    float4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int64_t slot = slot0 + (int64_t)min(s0 + j, a.n_split - 1) * rows;
+      ml[j] = *(const float2*)(a.ws_ml + 2 * slot);
+      v[j] = *(const float4*)(a.ws_o + slot * D + d);
+    }
+    float mb = M;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (s0 + j < a.n_split) mb = fmaxf(mb, ml[j].x);
+    const float al = __builtin_amdgcn_exp2f(M - mb);
+    M = mb;
+    L *= al;
+    acc.x *= al; acc.y *= al; acc.z *= al; acc.w *= al;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float w = s0 + j < a.n_split ? __builtin_amdgcn_exp2f(ml[j].x - mb) : 0.0f;
+      L = fmaf(ml[j].y, w, L);
+      acc.x = fmaf(v[j].x, w, acc.x);
+      acc.y = fmaf(v[j].y, w, acc.y);
+      acc.z = fmaf(v[j].z, w, acc.z);
+      acc.w = fmaf(v[j].w, w, acc.w);
+    }
   }
-  const float v = L > 0.0f ? acc / L : 0.0f;
-  uint16_t* orow = a.out + (int64_t)b * a.os_b + (int64_t)head * a.os_h + (int64_t)s * a.os_s;
-  orow[d] = F16 ? (uint16_t)f32_to_f16_bits(v) : (uint16_t)f32_to_bf16_bits(v);
+  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  const uint32_t w0 = pack2<F16>(acc.x * inv, acc.y * inv), w1 = pack2<F16>(acc.z * inv, acc.w * inv);
+  store4(a.out + (int64_t)b * a.os_b + (int64_t)head * a.os_h + (int64_t)s * a.os_s + d, w0, w1, a.o_vec);
 }
 
-template <int D, bool F16, int RB, int NW>
+template <int D, bool F16, int RB>
 void launch_prefill(const PrefillArgs& a, bool s_f16, dim3 grid, hipStream_t st) {
-  const dim3 block(64 * NW);
+  const dim3 block(256);
   if (a.bt) {
-    if (s_f16) hipLaunchKernelGGL((prefill_attn_kernel<D, F16, true, RB, true, NW>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((prefill_attn_kernel<D, F16, false, RB, true, NW>), grid, block, 0, st, a);
+    if (s_f16) hipLaunchKernelGGL((prefill_attn_kernel<D, F16, true, RB, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((prefill_attn_kernel<D, F16, false, RB, true>), grid, block, 0, st, a);
   } else {
-    if (s_f16) hipLaunchKernelGGL((prefill_attn_kernel<D, F16, true, RB, false, NW>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((prefill_attn_kernel<D, F16, false, RB, false, NW>), grid, block, 0, st, a);
+    if (s_f16) hipLaunchKernelGGL((prefill_attn_kernel<D, F16, true, RB, false>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((prefill_attn_kernel<D, F16, false, RB, false>), grid, block, 0, st, a);
   }
 }
 
 template <int D, bool F16>
-void launch_prefill_rb(const PrefillArgs& a, bool s_f16, int rb, int nw, dim3 grid, hipStream_t st) {
-  if constexpr (D == 128) {
-    if (nw == 8) launch_prefill<D, F16, 2, 8>(a, s_f16, grid, st);
-    else if (rb == 2) launch_prefill<D, F16, 2, 4>(a, s_f16, grid, st);
-    else launch_prefill<D, F16, 1, 4>(a, s_f16, grid, st);
-  } else {
-    if (rb == 2) launch_prefill<D, F16, 2, 4>(a, s_f16, grid, st);
-    else launch_prefill<D, F16, 1, 4>(a, s_f16, grid, st);
-  }
-  if (a.n_split > 1) {
-    const int rows = kWaveRows * nw * rb;
-    const int64_t n = (int64_t)grid.x / a.n_split * rows;
-    hipLaunchKernelGGL((prefill_merge_kernel<D, F16>), dim3((unsigned)n), dim3(D), 0, st, a, rows);
-  }
+void launch_merge(const PrefillArgs& a, int rows, hipStream_t st) {
+  const int64_t n = (int64_t)a.n_units * a.row_blocks * (rows / (1024 / D));
+  hipLaunchKernelGGL((prefill_merge_kernel<D, F16>), dim3((unsigned)n), dim3(256), 0, st, a, rows);
 }
 
-// Launch plan: waves per workgroup (nw), rows per workgroup (nw waves of rb
+template <int D, bool F16>
+void launch_prefill_rb(const PrefillArgs& a, bool s_f16, int rb, dim3 grid, hipStream_t st) {
+  if (rb == 2) launch_prefill<D, F16, 2>(a, s_f16, grid, st);
+  else launch_prefill<D, F16, 1>(a, s_f16, grid, st);
+  if (a.n_split > 1) launch_merge<D, F16>(a, kWaveRows * 4 * rb, st);
+}
+
+// One group of units on the staged route: images, attention, merge.
+template <int D, bool F16>
+void launch_staged(const PrefillArgs& a, bool s_f16, int nw, hipStream_t st) {
+  constexpr int TPB = 256 / D;
+  const dim3 sg((unsigned)((a.tiles + TPB - 1) / TPB), (unsigned)a.n_units);
+  if (a.tiles > 0) {
+    if (s_f16) hipLaunchKernelGGL((stage_kv_kernel<D, F16, true>), sg, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((stage_kv_kernel<D, F16, false>), sg, dim3(256), 0, st, a);
+  }
+  const dim3 grid((unsigned)((int64_t)a.n_units * a.row_blocks * a.n_split));
+  if (nw == 8) hipLaunchKernelGGL((prefill_staged_kernel<D, F16, 8>), grid, dim3(512), 0, st, a);
+  else hipLaunchKernelGGL((prefill_staged_kernel<D, F16, 4>), grid, dim3(256), 0, st, a);
+  if (a.n_split > 1) launch_merge<D, F16>(a, 32 * nw, st);
+}
+
+// Launch plan of the unstaged kernel: rows per workgroup (four waves of rb
 // 16-row blocks), row blocks, and the split over keys. Two row blocks per
-// wave once that still gives a workgroup of four waves per CU of a 256-CU
-// device. D = 128 with two row blocks takes eight waves per workgroup (one
-// workgroup of 256 rows per CU) once that still gives a workgroup per CU.
-// Below 512 workgroups of four waves (two per CU), splits of at least 512
-// keys bring the launch to ~512.
+// wave once that still gives a workgroup per CU of a 256-CU device. A launch
+// of fewer workgroups splits the keys. A tile takes a lone workgroup of a CU
+// about 1.3 us, and two workgroups of a CU together longer, so the target is
+// one workgroup per CU with splits of at least two tiles (D = 128, 8 KV heads,
+// 8 query positions at GQA 4: 1K keys 8 splits 12.8 us, 4 splits 15.2, 2
+// splits 20.8; 16K keys 32 splits 26.8 us, 64 splits 31.0); where that
+// leaves splits of over 1024 keys the launch is long enough to fill 512
+// workgroup slots (two per CU) instead.
 struct PrefillPlan {
-  int rb, nw, n_split;
+  int rb, n_split;
   int64_t row_blocks;
 };
 
-PrefillPlan prefill_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D) {
+PrefillPlan prefill_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk) {
   const int64_t ratio = Hq / Hkv;
   const int64_t rows = Sq * ratio;
   PrefillPlan p;
   p.rb = B * Hkv * ((rows + 8 * kWaveRows - 1) / (8 * kWaveRows)) >= 256 ? 2 : 1;
-  p.nw = (D == 128 && p.rb == 2 && B * Hkv * ((rows + 16 * kWaveRows - 1) / (16 * kWaveRows)) >= 256) ? 8 : 4;
-  const int64_t wg_rows = kWaveRows * p.nw * p.rb;
+  const int64_t wg_rows = kWaveRows * 4 * p.rb;
   p.row_blocks = (rows + wg_rows - 1) / wg_rows;
   const int64_t n_wg = B * Hkv * p.row_blocks;
   int64_t ns = 1;
-  if (p.nw == 4 && n_wg > 0 && n_wg < 512) {
-    ns = (512 + n_wg - 1) / n_wg;
-    ns = std::min<int64_t>(ns, std::max<int64_t>(1, Sk / 512));
+  if (n_wg > 0 && n_wg < 512) {
+    ns = std::min<int64_t>((256 + n_wg - 1) / n_wg, std::max<int64_t>(1, Sk / 128));
+    if (Sk > 1024 * ns) ns = std::min<int64_t>((512 + n_wg - 1) / n_wg, std::max<int64_t>(1, Sk / 512));
     ns = std::min<int64_t>(ns, 64);
   }
   p.n_split = (int)ns;
@@ -609,7 +1089,58 @@ PrefillPlan prefill_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t
 
 int64_t prefill_ws_bytes(const PrefillPlan& p, int64_t B, int64_t Hkv, int64_t D) {
   if (p.n_split <= 1) return 0;
-  return B * Hkv * p.row_blocks * p.n_split * (kWaveRows * p.nw * p.rb) * (D + 2) * 4;
+  return B * Hkv * p.row_blocks * p.n_split * (kWaveRows * 4 * p.rb) * (D + 2) * 4;
+}
+
+// Plan of the staged route. Units go in groups whose images fit kStageBytes
+// (the 256 MB Infinity Cache holds them then, and the workspace stays
+// bounded); a unit whose images alone do not fit (over 512K keys at D = 128)
+// is not staged. Eight waves (256 rows) per workgroup, one workgroup per CU,
+// once a group fills the device with them: an image then crosses from L2 once
+// per 256 rows; else four waves, two workgroups per CU. The split over keys is
+// the one with the shortest estimate: rounds of resident workgroups times a
+// workgroup's tiles (plus about four tiles of prologue and epilogue), plus
+// the merge (its launch and the partials' traffic, in tile times).
+struct StagedPlan {
+  int nw, n_split;       // nw = 0: not staged
+  int64_t group, row_blocks, img_bytes, part_rows;  // img_bytes: one unit's; part_rows: partial rows of a group
+};
+
+constexpr int64_t kStageBytes = int64_t(256) << 20;
+// Where staging starts to pay: the images cost a launch and 32 bytes of
+// traffic per key and dim pair, once per unit, and every 128 rows save one
+// dequantization of them. Measured, staged against not (us; 8 KV heads, D =
+// 128): 2K keys 1024 rows 38.1 / 35.9, 2048 rows 44.8 / 50.4; 4K keys 512 rows
+// 37.9 / 37.4, 1024 rows 45.6 / 52; 16K keys 128 rows 44.2 / 37.9, 256 rows
+// 48.7 / 52, 2048 rows 161 / 274; 32 units, 1K keys, 512 rows 35.9 / 37.6.
+constexpr int64_t kStagedMinRows = 256;
+constexpr int64_t kStagedMinWork = int64_t(1) << 24;  // units * rows * keys
+
+StagedPlan staged_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D) {
+  StagedPlan p = {0, 1, 0, 0, 0, 0};
+  const int64_t rows = Sq * (Hq / Hkv), units = B * Hkv, tiles = (Sk + kKeys - 1) / kKeys;
+  p.img_bytes = tiles * D * 256;
+  if (rows < kStagedMinRows || units * rows * Sk < kStagedMinWork || tiles == 0 || p.img_bytes > kStageBytes) return p;
+  p.group = std::min<int64_t>(std::min<int64_t>(units, 32768), kStageBytes / p.img_bytes);
+  p.nw = p.group * ((rows + 255) / 256) >= 256 ? 8 : 4;
+  p.row_blocks = (rows + 32 * p.nw - 1) / (32 * p.nw);
+  const int64_t n_wg = p.group * p.row_blocks, slots = p.nw == 8 ? 256 : 512;
+  double best = 0.0;
+  for (int64_t ns = 1; ns <= std::min<int64_t>(16, std::max<int64_t>(1, tiles / 8)); ++ns) {
+    const double rounds = (double)((n_wg * ns + slots - 1) / slots);
+    double cost = rounds * ((double)tiles / (double)ns + 4.0);
+    if (ns > 1) cost += 4.0 + (double)(n_wg * ns * 32 * p.nw) * (double)D * 8.0 / 4.0e6;
+    if (ns == 1 || cost < best) {
+      best = cost;
+      p.n_split = (int)ns;
+    }
+  }
+  p.part_rows = p.n_split > 1 ? n_wg * p.n_split * 32 * p.nw : 0;
+  return p;
+}
+
+int64_t staged_ws_bytes(const StagedPlan& p, int64_t D) {
+  return p.nw ? p.group * p.img_bytes + p.part_rows * (D + 2) * 4 : 0;
 }
 
 }  // namespace
@@ -676,13 +1207,16 @@ int prefill_impl(const void* q, int q_dtype, const int64_t* q_strides, const voi
   if (B == 0 || Sq == 0) return KVQ_OK;
   KVQ_CHECK_ARG(q && out && (Sk == 0 || (k_packed && k_scales && v_packed && v_scales)),
                 "kvq_prefill_attn: null data pointer");
-  PrefillPlan plan = prefill_plan(B, Hq, Hkv, Sq, Sk, D);
-  // the split over keys needs the workspace; without one the launch is unsplit
+  // the staged route and the split over keys need the workspace; without
+  // enough of it the launch is unstaged, then unsplit
+  StagedPlan sp = staged_plan(B, Hq, Hkv, Sq, pg && pg->bt_cols == 0 ? 0 : Sk, D);
+  if (workspace == nullptr || workspace_bytes < staged_ws_bytes(sp, D) || (uintptr_t)workspace % 16 != 0) sp.nw = 0;
+  PrefillPlan plan = prefill_plan(B, Hq, Hkv, Sq, Sk);
   const int64_t need = prefill_ws_bytes(plan, B, Hkv, D);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) plan.n_split = 1;
   const int rb = plan.rb;
-  const int64_t row_blocks = plan.row_blocks;
-  const int64_t n_wg = B * Hkv * row_blocks * plan.n_split;
+  const int64_t row_blocks = sp.nw ? sp.row_blocks : plan.row_blocks;
+  const int64_t n_wg = sp.nw ? sp.group * row_blocks * sp.n_split : B * Hkv * row_blocks * plan.n_split;
   KVQ_CHECK_ARG(n_wg < (1ll << 31) && Sq < (1ll << 30) && Sk < (1ll << 30), "kvq_prefill_attn: too large");
 
   PrefillArgs a;
@@ -708,20 +1242,51 @@ int prefill_impl(const void* q, int q_dtype, const int64_t* q_strides, const voi
   a.n_blocks = pg ? (int)pg->n_blocks : 0;
   a.page_shift = page_shift;
   if (pg && pg->bt_cols == 0) a.Sk = 0;
-  a.n_split = plan.n_split;
-  a.ws_o = plan.n_split > 1 ? (float*)workspace : nullptr;
-  a.ws_ml = plan.n_split > 1 ? (float*)workspace + B * Hkv * row_blocks * plan.n_split * (kWaveRows * plan.nw * rb) * D
-                              : nullptr;
-
-  const dim3 grid((unsigned)n_wg);
+  // 16-byte query and code pieces, 8-byte output pieces where every row is
+  // aligned for them
+  auto multiples = [](const void* p, int64_t bytes, const int64_t* st, int64_t n) {
+    return (uintptr_t)p % bytes == 0 && st[0] % n == 0 && st[1] % n == 0 && st[2] % n == 0;
+  };
+  a.q_vec = multiples(q, 16, q_strides, 8) ? 1 : 0;
+  a.o_vec = multiples(out, 8, out_strides, 4) ? 1 : 0;
+  a.kv_vec = multiples(k_packed, 16, kp_strides, 16) && multiples(v_packed, 4, vp_strides, 4) ? 1 : 0;
+  a.u0 = 0;
+  a.n_units = (int)(B * Hkv);
+  a.tiles = 0;
+  a.img = nullptr;
   hipStream_t st = (hipStream_t)stream;
   const bool f16 = q_dtype == KVQ_F16, s_f16 = scale_dtype == KVQ_F16;
+  if (sp.nw) {
+    a.n_split = sp.n_split;
+    a.tiles = (a.Sk + kKeys - 1) / kKeys;
+    a.img = (uint4*)workspace;
+    a.ws_o = sp.n_split > 1 ? (float*)((char*)workspace + sp.group * sp.img_bytes) : nullptr;
+    a.ws_ml = sp.n_split > 1 ? a.ws_o + sp.part_rows * D : nullptr;
+    for (int64_t u0 = 0; u0 < B * Hkv; u0 += sp.group) {
+      a.u0 = (int)u0;
+      a.n_units = (int)std::min<int64_t>(sp.group, B * Hkv - u0);
+      if (D == 128) {
+        if (f16) launch_staged<128, true>(a, s_f16, sp.nw, st);
+        else launch_staged<128, false>(a, s_f16, sp.nw, st);
+      } else {
+        if (f16) launch_staged<64, true>(a, s_f16, sp.nw, st);
+        else launch_staged<64, false>(a, s_f16, sp.nw, st);
+      }
+    }
+    KVQ_CHECK_LAUNCH("kvq_prefill_attn");
+    return KVQ_OK;
+  }
+  a.n_split = plan.n_split;
+  a.ws_o = plan.n_split > 1 ? (float*)workspace : nullptr;
+  a.ws_ml = plan.n_split > 1 ? (float*)workspace + B * Hkv * row_blocks * plan.n_split * (kWaveRows * 4 * rb) * D : nullptr;
+
+  const dim3 grid((unsigned)n_wg);
   if (D == 128) {
-    if (f16) launch_prefill_rb<128, true>(a, s_f16, rb, plan.nw, grid, st);
-    else launch_prefill_rb<128, false>(a, s_f16, rb, plan.nw, grid, st);
+    if (f16) launch_prefill_rb<128, true>(a, s_f16, rb, grid, st);
+    else launch_prefill_rb<128, false>(a, s_f16, rb, grid, st);
   } else {
-    if (f16) launch_prefill_rb<64, true>(a, s_f16, rb, plan.nw, grid, st);
-    else launch_prefill_rb<64, false>(a, s_f16, rb, plan.nw, grid, st);
+    if (f16) launch_prefill_rb<64, true>(a, s_f16, rb, grid, st);
+    else launch_prefill_rb<64, false>(a, s_f16, rb, grid, st);
   }
   KVQ_CHECK_LAUNCH("kvq_prefill_attn");
   return KVQ_OK;
@@ -754,7 +1319,15 @@ extern "C" int64_t kvq_prefill_attn_workspace_bytes(int64_t B, int64_t Hq, int64
     return KVQ_EINVAL;
   }
   if (B == 0 || Sq == 0) return 0;
-  return prefill_ws_bytes(prefill_plan(B, Hq, Hkv, Sq, Sk, D), B, Hkv, D);
+  return prefill_ws_bytes(prefill_plan(B, Hq, Hkv, Sq, Sk), B, Hkv, D);
+}
+
+extern "C" int64_t kvq_prefill_attn_staged_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
+                                                           int64_t D, int64_t Sk) {
+  const int64_t n = kvq_prefill_attn_workspace_bytes(B, Hq, Hkv, Sq, D, Sk);
+  if (n < 0 || B == 0 || Sq == 0) return n;
+  const int64_t staged = staged_ws_bytes(staged_plan(B, Hq, Hkv, Sq, Sk, D), D);
+  return std::max(staged, n);
 }
 
 extern "C" int kvq_prefill_attn_paged(const void* q, int q_dtype, const int64_t* q_strides,

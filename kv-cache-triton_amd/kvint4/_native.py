@@ -43,6 +43,7 @@ EXPORTED_SYMBOLS = (
     "kvq_decode_step_paged",
     "kvq_prefill_attn",
     "kvq_prefill_attn_workspace_bytes",
+    "kvq_prefill_attn_staged_workspace_bytes",
     "kvq_prefill_attn_paged",
 )
 
@@ -112,6 +113,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     ]
     lib.kvq_prefill_attn_workspace_bytes.restype = _i64
     lib.kvq_prefill_attn_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64, _i64, _i64]
+    lib.kvq_prefill_attn_staged_workspace_bytes.restype = _i64
+    lib.kvq_prefill_attn_staged_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64, _i64, _i64]
     lib.kvq_prefill_attn.restype = _i32
     lib.kvq_prefill_attn.argtypes = [
         _vp, _i32, _i64p,

@@ -260,9 +260,6 @@ class _Workspaces:
 
 
 _workspaces = _Workspaces()
-# prefill split partials: a separate buffer, so that they never overwrite the
-# decode kernels' arrival counters
-_prefill_workspaces = _Workspaces()
 
 
 def decode_workspace_bytes(B: int, Hq: int, Hkv: int, D: int, q_dtype: torch.dtype,
@@ -285,15 +282,23 @@ def using_workspace(buf: torch.Tensor):
     return _workspaces.using(buf)
 
 
-def _prefill_ws(q: torch.Tensor, Hkv: int, Sk: int, stream: int) -> tuple:
+def _prefill_ws(q: torch.Tensor, Hkv: int, Sk: int) -> tuple:
+    """(tensor, pointer, bytes) of the prefill kernels' scratch: the operand
+    images of the staged route (at most 256 MiB, whatever the batch) and the
+    partials of a split over keys. It needs no initialisation and is only used
+    by launches enqueued on the current stream while the caller holds it, so
+    it comes from the caching allocator and goes back to it with the call
+    (under graph capture: the graph's own pool)."""
     B, Hq, Sq, D = q.shape
-    n = nat.lib().kvq_prefill_attn_workspace_bytes(B, Hq, Hkv, Sq, D, Sk)
+    n = nat.lib().kvq_prefill_attn_staged_workspace_bytes(B, Hq, Hkv, Sq, D, Sk)
     if n < 0:
-        nat.check(int(n), "kvq_prefill_attn_workspace_bytes")
+        nat.check(int(n), "kvq_prefill_attn_staged_workspace_bytes")
     if n == 0:
-        return None, 0
-    ws = _prefill_workspaces.get(q.device, stream, n)
-    return ws.data_ptr(), ws.numel()
+        return None, None, 0
+    ws = torch.empty(n, dtype=torch.uint8, device=q.device)
+    return ws, ws.data_ptr(), n
+
+
 _cu_count: dict[int, int] = {}
 
 
@@ -411,7 +416,7 @@ def prefill_attention(
     lib = nat.lib()
     with nat.device_of(q):
         stream = nat.stream_handle(q.device)
-        ws_ptr, ws_len = _prefill_ws(q, n_kv_heads, Sk, stream)
+        ws, ws_ptr, ws_len = _prefill_ws(q, n_kv_heads, Sk)
         rc = lib.kvq_prefill_attn(
             q.data_ptr(), nat.DTYPE_CODE[q.dtype], nat.i64_array(q.stride()),
             k_packed.data_ptr(), nat.i64_array(k_packed.stride()[:3]),
@@ -893,7 +898,7 @@ def prefill_attention_paged(
     lib = nat.lib()
     with nat.device_of(q):
         stream = nat.stream_handle(q.device)
-        ws_ptr, ws_len = _prefill_ws(q, n_kv_heads, seq_len, stream)
+        ws, ws_ptr, ws_len = _prefill_ws(q, n_kv_heads, seq_len)
         rc = lib.kvq_prefill_attn_paged(
             q.data_ptr(), nat.DTYPE_CODE[q.dtype], nat.i64_array(q.stride()),
             k_pool.data_ptr(), nat.i64_array(k_pool.stride()[:2]),
