@@ -36,8 +36,9 @@ struct QuantArgs {
   int x_dtype, scale_dtype;
   PageMap pm;  // pm.paged: packed/scales are pools (ps_b = ss_b = 0)
   // row -> (b, h, s) and thread -> (row, chunk) without runtime divides
-  // (vector path; rows * D / 8 < 2^32)
+  // (vector path; rows * cpr < 2^32)
   FastDiv div_s, div_h, div_cpr;
+  uint32_t cpr;  // 8-element chunks per row (vector path)
 };
 
 // Destination row of (b, position), or -1 where it does not exist: the
@@ -104,9 +105,12 @@ __global__ __launch_bounds__(256) void quantize_kernel(const QuantArgs a) {
 // absmax is all-reduced across those lanes with DPP (quad xor 1, quad xor 2,
 // half-row mirror, row mirror), every lane divides its own 8 elements by the
 // group scale and packs them into one 4-byte store; the group's first lane
-// stores the scale. Taken when G is 8..128 (power of two), G divides D, x rows
-// have unit inner stride and 16-byte aligned starts, and packed rows are
-// 4-byte aligned; everything else takes quantize_kernel.
+// stores the scale. A last group that D only partly fills is padded with
+// chunks of zeros. Taken when G is 8..128 (power of two),
+// 8 divides D, x rows have unit inner stride and 16-byte aligned starts, and
+// packed rows are 4-byte aligned; everything else takes quantize_kernel (one
+// thread per group, byte stores: [2, 32, 3001, 80] bf16 at G = 32 took it 92 us
+// and takes this one 14.4 us).
 
 // The vector kernels stream every byte once, so their bulk accesses carry
 // the nontemporal hint (the `nt` bit): the quantizer's input loads and code
@@ -131,7 +135,7 @@ __device__ __forceinline__ float dpp_f(float v) {
 // need the positions. Placing each row only after the previous row's loads
 // had arrived cost a memory round trip per row (2.6 us of a 4.8 us launch
 // for one token of 8 heads). Index arithmetic is 32-bit (the host takes this
-// path only when rows * D / 8 < 2^32).
+// path only when rows * cpr < 2^32).
 // Rows per thread of the vector quantize / dequantize kernels: four for
 // large launches (more loads in flight per lane), one for launches of at
 // most kSmallChunks 8-element chunks. A small launch (a decode token's K or
@@ -143,13 +147,17 @@ constexpr int64_t kSmallChunks = 256 * 1024;
 template <int XDT, int LPG, int RPT>  // LPG = lanes per group = G / 8
 __global__ __launch_bounds__(256) void quantize_vec_kernel(const QuantArgs a) {
   const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t cpr = (uint32_t)a.D >> 3;  // chunks per row
+  const uint32_t cpr = a.cpr;  // chunks per padded row (ngroups * G / 8)
   const uint32_t rows = (uint32_t)a.rows;
   const uint32_t rq = (rows + RPT - 1) / RPT;
   const bool slot = idx < rq * cpr;
   const uint32_t r0 = slot ? fdiv(idx, a.div_cpr) : 0u;
   const uint32_t ch = slot ? idx - r0 * cpr : 0u;
   const uint32_t S = (uint32_t)a.S, H = (uint32_t)a.H;
+  // a chunk of the last group's padding (D not a multiple of G) reads its
+  // row's first chunk and is zeroed
+  const bool pad = 8 * ch >= (uint32_t)a.D;
+  const uint32_t chl = pad ? 0u : ch;
 
   constexpr int NW = XDT == KVQ_F32 ? 2 : 1;  // 16-byte loads per chunk
   bool live[RPT];
@@ -164,7 +172,7 @@ __global__ __launch_bounds__(256) void quantize_vec_kernel(const QuantArgs a) {
     ss[k] = rw - bh * S;
     bb[k] = fdiv(bh, a.div_h);
     hh[k] = bh - bb[k] * H;
-    const int64_t xoff = (int64_t)bb[k] * a.xs_b + (int64_t)hh[k] * a.xs_h + (int64_t)ss[k] * a.xs_s + 8 * ch;
+    const int64_t xoff = (int64_t)bb[k] * a.xs_b + (int64_t)hh[k] * a.xs_h + (int64_t)ss[k] * a.xs_s + 8 * chl;
 #pragma unroll
     for (int n = 0; n < NW; ++n)
       raw[k][n] = __builtin_bit_cast(
@@ -211,6 +219,8 @@ __global__ __launch_bounds__(256) void quantize_vec_kernel(const QuantArgs a) {
   }
 #pragma unroll
   for (int k = 0; k < RPT; ++k) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[k][e] = pad ? 0.0f : x[k][e];
     float amax = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(x[k][e]));
@@ -285,6 +295,7 @@ struct DequantArgs {
   int scale_dtype, out_dtype;
   PageMap pm;  // pm.paged: packed/scales are pools (ps_b = ss_b = 0)
   FastDiv div_s, div_h, div_cpr;  // as in QuantArgs (vector path)
+  FastDiv div_gc;                 // chunk -> group: division by G / 8
 };
 
 __global__ __launch_bounds__(256) void dequantize_kernel(const DequantArgs a) {
@@ -318,9 +329,11 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const DequantArgs a) {
 
 // Vector path: one thread per 8 consecutive elements of a row (one 4-byte
 // code word and its group's scale in, one 16-byte store of 16-bit outputs or
-// two of fp32 out). Taken when G is a multiple of 8 dividing d_out (=
-// groups * G), packed rows are 4-byte aligned and output rows have unit
-// inner stride and 16-byte aligned starts.
+// two of fp32 out). Taken when G and d_out are multiples of 8 (d_out may end
+// inside the last group: its other chunks are not read), packed rows are
+// 4-byte aligned and output rows have unit inner stride and 16-byte aligned
+// starts (d_out = 80 of G = 32, [2, 32, 3001] rows to bf16: 123 us one lane
+// per group, 11.4 us here).
 template <int ODT, int RPT>
 __global__ __launch_bounds__(256) void dequantize_vec_kernel(const DequantArgs a) {
   const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -357,7 +370,7 @@ __global__ __launch_bounds__(256) void dequantize_vec_kernel(const DequantArgs a
     for (int k = 0; k < RPT; ++k) {
       const int64_t b = bb[k], h = hh[k], rr = r[k] < 0 ? 0 : r[k];
       w[k] = *(const uint32_t*)(a.packed + b * a.ps_b + h * a.ps_h + rr * a.ps_s + 4 * ch);
-      si[k] = b * a.ss_b + h * a.ss_h + rr * a.ss_s + (8 * ch) / a.G;
+      si[k] = b * a.ss_b + h * a.ss_h + rr * a.ss_s + fdiv(ch, a.div_gc);
     }
     load_n_as_f32<RPT>(a.scales, si, a.scale_dtype, sc);
   }
@@ -482,21 +495,23 @@ int quantize_impl(const char* who, const void* x, int x_dtype, const int64_t* x_
   a.pm = pm;
   a.div_s = make_fastdiv((uint32_t)S);
   a.div_h = make_fastdiv((uint32_t)H);
-  a.div_cpr = make_fastdiv((uint32_t)std::max<int64_t>(1, D / 8));
+  const int64_t cpr = ngroups * group_size / 8;
+  a.cpr = (uint32_t)cpr;
+  a.div_cpr = make_fastdiv((uint32_t)std::max<int64_t>(1, cpr));
 
   hipStream_t st = (hipStream_t)stream;
   const int lpg = (int)(group_size / 8);
   const int64_t esz = dtype_size(x_dtype);
   const bool vec = group_size % 8 == 0 && group_size <= 128 && (lpg & (lpg - 1)) == 0 &&
-                   D % group_size == 0 && a.xs_d == 1 &&
+                   D % 8 == 0 && a.xs_d == 1 &&
                    (uintptr_t)x % 16 == 0 && (a.xs_b * esz) % 16 == 0 && (a.xs_h * esz) % 16 == 0 &&
                    (a.xs_s * esz) % 16 == 0 &&
                    (uintptr_t)packed % 4 == 0 && a.ps_b % 4 == 0 && a.ps_h % 4 == 0 && a.ps_s % 4 == 0 &&
-                   rows * (D / 8) < (1ll << 32) - 256 * kQuantRows;
+                   rows * cpr < (1ll << 32) - 256 * kQuantRows;
   if (vec) {
-    const bool small = rows * (D / 8) <= kSmallChunks;
+    const bool small = rows * cpr <= kSmallChunks;
     const int rpt = small ? 1 : kQuantRows;
-    const int64_t total = (rows + rpt - 1) / rpt * (D / 8);
+    const int64_t total = (rows + rpt - 1) / rpt * cpr;
     const dim3 grid((unsigned)((total + 255) / 256));
     switch (x_dtype) {
       case KVQ_BF16: small ? launch_qvec<KVQ_BF16, 1>(lpg, grid, st, a) : launch_qvec<KVQ_BF16, kQuantRows>(lpg, grid, st, a); break;
@@ -549,9 +564,10 @@ int dequantize_impl(const void* packed, const int64_t* packed_strides,
   a.div_s = make_fastdiv((uint32_t)S);
   a.div_h = make_fastdiv((uint32_t)H);
   a.div_cpr = make_fastdiv((uint32_t)std::max<int64_t>(1, d_out / 8));
+  a.div_gc = make_fastdiv((uint32_t)std::max<int64_t>(1, group_size / 8));
 
   const int64_t oes = dtype_size(out_dtype);
-  const bool vec = group_size % 8 == 0 && d_out == num_groups * group_size && a.os_d == 1 &&
+  const bool vec = group_size % 8 == 0 && d_out % 8 == 0 && a.os_d == 1 &&
                    (uintptr_t)out % 16 == 0 && (a.os_b * oes) % 16 == 0 && (a.os_h * oes) % 16 == 0 &&
                    (a.os_s * oes) % 16 == 0 && (uintptr_t)packed % 4 == 0 && a.ps_b % 4 == 0 &&
                    a.ps_h % 4 == 0 && a.ps_s % 4 == 0 && rows * (d_out / 8) < (1ll << 32) - 256 * kQuantRows;
