@@ -1578,6 +1578,295 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
 }
 
 // ===========================================================================
+// fp32 query blocks (prompts, prompt chunks, speculative blocks of fp32
+// models) on the fp32 matrix instructions: 16 query rows per workgroup, one
+// split. The VALU kernel below takes two fp32 rows per workgroup, so a block
+// of R rows streams and dequantizes the whole cache R / 2 times per KV head
+// (a 1000-token GPT-2 prompt: 500 times for each of 12 heads, 173 us); here it
+// is R / 16 times, and keys past a chunk's last admissible one are not read.
+// The four waves take 64-key tiles round-robin and are folded at the end, as
+// in the other kernels: a prompt's 63 chunks x 12 heads then give 756
+// workgroups of at most four tiles per wave, about three waves per SIMD.
+//
+// v_mfma_f32_16x16x4f32 (lane l: n = l % 16, g = l / 16): A[i][k] at lane i +
+// 16 k, B[k][j] at lane j + 16 k, C[i][j] at lane j + 16 (i / 4), register
+// i % 4; exact fp32 products and sums.
+//   S^T = K Q^T  per 16-key block: lane (i, g) holds dims [g D / 4, (g + 1)
+//     D / 4) of key i (one vector load of its code row, one scale), step e
+//     multiplies dim g D / 4 + e of all four lane groups.
+//   O^T += V^T P^T  step (block, r) covers keys 16 block + 4 g + r, whose
+//     weights are register r of the block's scores in the lanes that hold
+//     them: the weights never move. A: lane (i, g) holds V dims [i D / 16,
+//     (i + 1) D / 16) of that key; product db covers dims i D / 16 + db.
+// K and V are dequantized as (n - 8) * scale in fp32 (exact for 16-bit
+// scales), two instructions an element. Bound by instruction issue: a tile's
+// 128 matrix instructions (D = 64) take 4096 cycles, and the VALU beside them
+// nearly as many where a SIMD has few waves. The 1000-token prompt takes 34
+// us (173 on the VALU kernel); 36 with a four-bit extract per element, 47
+// with eight waves per workgroup (three waves per SIMD then leave one
+// workgroup per CU), 44 without the mixed chunk order below.
+constexpr int kBlockRows = 16;
+constexpr int kBlockWaves = 4;
+#ifndef F32MR
+#define F32MR 8
+#endif
+constexpr int kF32BlockMinRows = F32MR;
+
+template <int D, bool PAGED>
+__global__ __launch_bounds__(64 * kBlockWaves) void decode_attn_f32_block_kernel(const AttnArgs a) {
+  constexpr int ROWS = kBlockRows, NW = kBlockWaves;
+  constexpr int KD = D / 4;   // K dims per lane
+  constexpr int VD = D / 16;  // V dims per lane
+  constexpr int KW = KD / 8;  // K code dwords per lane
+  __shared__ float o_lds[NW][ROWS][D];
+  __shared__ __attribute__((aligned(16))) float ml_lds[NW][ROWS][2];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  int unit, split;
+  if (!unit_and_split(a, unit, split)) return;
+  int b, kvh, rc;
+  unit_coords(a, unit, b, kvh, rc);
+  // a causal chunk's work grows with its index, and a CU takes every 256th
+  // unit or so: reversing the chunks of every other 256 units' heads gives a
+  // CU long and short ones
+  if ((((uint32_t)(unit - rc) >> 8) & 1u) == 0u) rc = a.row_chunks - 1 - rc;
+  int L = a.Sk;
+  if (a.seq_lens) L = a.seq_lens[b];
+  L = L < 0 ? 0 : (L < a.Sk ? L : a.Sk);
+
+  // this lane's query row and the keys it may attend: [0, lim)
+  const int rho = rc * ROWS + n;
+  const bool row_ok = rho < a.rows_total;
+  const int rho_c = row_ok ? rho : 0;
+  const int hq = (int)fdiv((uint32_t)rho_c, a.div_sq), qi = rho_c - hq * a.Sq;
+  int lim = a.causal ? L - a.Sq + qi + 1 : L;
+  lim = row_ok && lim > 0 ? lim : 0;
+  float qf[KD];
+  {
+    const float* q = (const float*)a.q + (int64_t)b * a.qs_b + (int64_t)(kvh * a.ratio + hq) * a.qs_h +
+                     (int64_t)qi * a.qs_s + (int64_t)(KD * g) * a.qs_d;
+    if (a.q_vec) {
+#pragma unroll
+      for (int e = 0; e < KD; e += 4) {
+        const float4 x = *(const float4*)(q + e);
+        qf[e] = x.x; qf[e + 1] = x.y; qf[e + 2] = x.z; qf[e + 3] = x.w;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < KD; ++e) qf[e] = q[(int64_t)e * a.qs_d];
+    }
+#pragma unroll
+    for (int e = 0; e < KD; ++e) qf[e] = row_ok ? qf[e] : 0.0f;
+  }
+  // keys any row of the chunk attends (wave-uniform)
+  int kend = lim;
+#pragma unroll
+  for (int m = 1; m < 16; m *= 2) kend = max(kend, __shfl_xor(kend, m));
+  kend = __builtin_amdgcn_readfirstlane(kend);
+  int ntiles = (kend + 63) / 64;
+  if constexpr (PAGED) {
+    if (a.n_blocks == 0) ntiles = 0;
+  }
+  const int32_t* bt_b = PAGED ? a.bt + (int64_t)b * a.bt_stride : nullptr;
+
+  const uint8_t* kp_bh = a.kp + (int64_t)b * a.kps_b + (int64_t)kvh * a.kps_h;
+  const uint8_t* vp_bh = a.vp + (int64_t)b * a.vps_b + (int64_t)kvh * a.vps_h;
+  const int s_esize = a.scale_dtype == KVQ_F32 ? 4 : 2;
+  const char* ks_bh = (const char*)a.ks + ((int64_t)b * a.kss_b + (int64_t)kvh * a.kss_h) * s_esize;
+  const char* vs_bh = (const char*)a.vs + ((int64_t)b * a.vss_b + (int64_t)kvh * a.vss_h) * s_esize;
+  const uint32_t kps = (uint32_t)a.kps_s, vps = (uint32_t)a.vps_s;
+  const uint32_t kss = (uint32_t)a.kss_s, vss = (uint32_t)a.vss_s;
+  const uint32_t gK = fdiv((uint32_t)(KD * g), a.div_g), gV = fdiv((uint32_t)(VD * n), a.div_g);
+  const int last_tok = L > 0 ? L - 1 : 0;
+
+  // raw codes and scales of a tile: K of keys 16 kb + n, V of keys 16 kb +
+  // 4 g + r. Keys past the sequence read its last row (inside the tile, hence
+  // in its page) and are masked; a paged tile without a block reads pool row 0
+  // and is masked.
+  uint32_t kw[4][KW], vw[4][4];
+  float ksc[4], vsc[4][4];
+  bool have = false;  // a block holds the tile in kw / vw
+  auto load_tile = [&](int tile) {
+    const int t0 = 64 * tile;
+    uint32_t dl = 0u;
+    bool ok = true;
+    if constexpr (PAGED) page_delta(a, bt_b, (uint32_t)t0, dl, ok);
+    have = ok;
+    auto row = [&](int t) -> uint32_t {
+      const uint32_t tc = (uint32_t)min(t, last_tok);
+      return ok ? tc + dl : 0u;
+    };
+    uint32_t kr[4], vr[4][4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      kr[kb] = row(t0 + 16 * kb + n);
+      const uint8_t* kp = kp_bh + (kr[kb] * kps + (uint32_t)(KD / 2) * (uint32_t)g);
+      if constexpr (KW == 2) {
+        const uint2 w = *(const uint2*)kp;
+        kw[kb][0] = w.x; kw[kb][1] = w.y;
+      } else {
+        const uint4 w = *(const uint4*)kp;
+        kw[kb][0] = w.x; kw[kb][1] = w.y; kw[kb][2] = w.z; kw[kb][3] = w.w;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        vr[kb][r] = row(t0 + 16 * kb + 4 * g + r);
+        const uint8_t* vp = vp_bh + (vr[kb][r] * vps + (uint32_t)(VD / 2) * (uint32_t)n);
+        if constexpr (VD == 4) vw[kb][r] = *(const uint16_t*)vp;
+        else vw[kb][r] = *(const uint32_t*)vp;
+      }
+    }
+    if (a.scale_dtype == KVQ_F32) {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        ksc[kb] = 0.0625f * ((const float*)ks_bh)[kr[kb] * kss + gK];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vsc[kb][r] = 0.0625f * ((const float*)vs_bh)[vr[kb][r] * vss + gV];
+      }
+    } else {
+      uint32_t kh[4], vh[4][4];
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        kh[kb] = ((const uint16_t*)ks_bh)[kr[kb] * kss + gK];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vh[kb][r] = ((const uint16_t*)vs_bh)[vr[kb][r] * vss + gV];
+      }
+      if (a.scale_dtype == KVQ_F16) {
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+          ksc[kb] = 0.0625f * f16_bits_to_f32(kh[kb]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) vsc[kb][r] = 0.0625f * f16_bits_to_f32(vh[kb][r]);
+        }
+      } else {
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+          ksc[kb] = 0.0625f * bf16_bits_to_f32(kh[kb]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) vsc[kb][r] = 0.0625f * bf16_bits_to_f32(vh[kb][r]);
+        }
+      }
+    }
+  };
+  // 16 (n - 8) in fp32 for nibble n = e of a code dword, from lo and hi: its
+  // even and odd nibbles, less 8, in the upper halves of signed bytes (one
+  // byte conversion; the scales carry the factor 1/16)
+  auto halves = [](uint32_t w, uint32_t& lo, uint32_t& hi) {
+    w ^= 0x88888888u;
+    lo = (w << 4) & 0xf0f0f0f0u;
+    hi = w & 0xf0f0f0f0u;
+    // (through an empty asm: with the mask visible the compiler folds it into
+    // each element's extract, two more instructions than the byte conversion)
+    asm("" : "+v"(lo), "+v"(hi));
+  };
+  auto code = [](uint32_t lo, uint32_t hi, int e) -> float {
+    return (float)(int)(int8_t)(((e & 1) ? hi : lo) >> (8 * (e >> 1)));
+  };
+
+  f32x4_t o[VD];
+#pragma unroll
+  for (int db = 0; db < VD; ++db) o[db] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  float m_run = kNeg, l_run = 0.0f;
+  for (int tile = wave; tile < ntiles; tile += NW) {
+    load_tile(tile);
+    f32x4_t st[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) st[kb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < KW; ++w) {
+      uint32_t lo[4], hi[4];
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        halves(kw[kb][w], lo[kb], hi[kb]);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb)
+          st[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(code(lo[kb], hi[kb], e) * ksc[kb], qf[8 * w + e], st[kb], 0, 0, 0);
+    }
+    // operands are converted a few instructions ahead of the product that
+    // reads them, between the products before it
+    __builtin_amdgcn_sched_group_barrier(0x002, 24, 0);
+#pragma unroll
+    for (int i = 0; i < 4 * KD; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+    }
+    // scores in base 2; excluded keys -inf (weight exactly 0)
+    const int klim = have ? lim - 64 * tile - 4 * g : 0;
+    float mx = -__builtin_inff();
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        st[kb][r] = 16 * kb + r < klim ? st[kb][r] * a.scale_log2 : -__builtin_inff();
+        mx = fmaxf(mx, st[kb][r]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(m_run, mx);
+    if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int db = 0; db < VD; ++db) o[db] *= alpha;
+    }
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float p = __builtin_amdgcn_exp2f(st[kb][r] - m_run);
+        l_run += p;
+        uint32_t lo, hi;
+        halves(vw[kb][r], lo, hi);
+#pragma unroll
+        for (int db = 0; db < VD; ++db)
+          o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(code(lo, hi, db) * vsc[kb][r], p, o[db], 0, 0, 0);
+      }
+  }
+
+  // wave partials -> LDS: o[db][j] is dim VD (4 g + j) + db of row n
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int db = 0; db < VD; ++db) o_lds[wave][n][VD * (4 * g + j) + db] = o[db][j];
+  float l_tot = l_run + __shfl_xor(l_run, 16);
+  l_tot += __shfl_xor(l_tot, 32);
+  if (g == 0) {
+    ml_lds[wave][n][0] = m_run;
+    ml_lds[wave][n][1] = l_tot;
+  }
+  __syncthreads();
+  for (int idx = tid; idx < ROWS * D / 4; idx += 64 * NW) {
+    const int r = idx / (D / 4), d = 4 * (idx % (D / 4));
+    float M = kNeg, Ls = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, ml_lds[w][r][0]);
+    float4 O = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = __builtin_amdgcn_exp2f(ml_lds[w][r][0] - M);
+      const float4 x = *(const float4*)&o_lds[w][r][d];
+      Ls = fmaf(ml_lds[w][r][1], f, Ls);
+      O.x = fmaf(x.x, f, O.x);
+      O.y = fmaf(x.y, f, O.y);
+      O.z = fmaf(x.z, f, O.z);
+      O.w = fmaf(x.w, f, O.w);
+    }
+    const int rr = rc * ROWS + r;
+    if (rr < a.rows_total) {
+      const bool any = Ls > 0.0f;  // a row without an admissible key yields zeros
+      store4_from_f32(a, out_index(a, b, kvh, rr, d), KVQ_F32, any ? O.x / Ls : 0.0f, any ? O.y / Ls : 0.0f,
+                      any ? O.z / Ls : 0.0f, any ? O.w / Ls : 0.0f);
+    }
+  }
+}
+
+// ===========================================================================
 // VALU kernel: fp32 queries (exact fp32 arithmetic) or fp32 scales.
 // Lane = token * (D/32) + chunk for QK (quad-reduced with DPP); V lanes own 8
 // output dims and four tokens per tile.
@@ -1995,6 +2284,7 @@ __global__ __launch_bounds__(256) void decode_attn_valu_kernel(const AttnArgs a)
 
 struct Plan {
   bool mfma;
+  bool f32_block;  // fp32 query block on decode_attn_f32_block_kernel (one split)
   int rows, row_chunks, n_units, n_split;
 };
 
@@ -2015,6 +2305,25 @@ static int64_t min_split_tokens(bool mfma, int64_t D) {
   return 128;
 }
 
+// Whether an fp32 query block runs on the 16-row matrix kernel (one split).
+// Its time is set by one workgroup's walk over the keys (about 3.8 us per 256
+// of them at D = 64, 6.8 at D = 128) until the device is full; the VALU
+// kernel's by the two-row chunks it streams the keys for (3e-5 us per chunk
+// and key at D = 64, 4.2e-5 at D = 128), split over keys. The lines are where
+// the two meet, whatever the key count: about 1024 rows over all heads at D =
+// 64, 1280 at D = 128 (measured, VALU / matrix, us: 12 heads of 64, 1K keys,
+// 64 positions 21.1 / 20.4, 128 positions 31.8 / 20.6, 4K keys 50 / 67 and
+// 78 / 68; 8 KV heads of 128, GQA 4, 1K keys, 32 positions 29.9 / 33.8, 64
+// positions 54 / 34.5). Up to 512 keys at D = 64, where the VALU kernel has
+// few splits, from 192 rows (512 keys: 8 positions 11.7 / 12.5, 16 positions
+// 15.0 / 12.4). A decode token (Sq = 1) stays on the VALU kernel, which also
+// appends, and so does a call that asks for splits.
+static bool use_f32_block(int64_t bh, int64_t rows_total, int64_t Sq, int64_t D, int64_t s_max, int q_dtype,
+                          int64_t n_split_req) {
+  if (q_dtype != KVQ_F32 || Sq < 2 || n_split_req > 1) return false;
+  return bh * rows_total >= (D == 64 ? (s_max <= 512 ? 192 : 1024) : 1280);
+}
+
 // Split-K plan: enough splits that B * Hkv * row_chunks * n_split workgroups
 // cover the CUs once (one resident workgroup per CU), no split shorter than
 // min_split_tokens of the longest sequence, at most kMaxSplit.
@@ -2024,8 +2333,12 @@ static int make_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t D, 
   if (!(D == 64 || D == 128)) return KVQ_EUNSUP;
   const int64_t rows_total = (Hq / Hkv) * Sq;
   p->mfma = use_mfma(q_dtype, scale_dtype);
+  p->f32_block = false;
   if (p->mfma) {
     p->rows = rows_total <= 4 ? 4 : 8;
+  } else if (use_f32_block(B * Hkv, rows_total, Sq, D, s_max, q_dtype, n_split_req)) {
+    p->f32_block = true;
+    p->rows = kBlockRows;
   } else {
     const int cap = q_dtype == KVQ_F32 ? 2 : 8;
     int r = 1;
@@ -2041,7 +2354,7 @@ static int make_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t D, 
   int64_t ns = n_split_req;
   if (ns <= 0) {
     const int64_t cus = std::max<int64_t>(1, num_cus);
-    ns = (cus + units - 1) / units;
+    ns = p->f32_block ? 1 : (cus + units - 1) / units;
   }
   ns = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(ns, max_split), kMaxSplit));
   if (units * ns > 0x7fffffffll || units * p->rows * D / 128 >= 0x7fffffffll) return KVQ_EUNSUP;
@@ -2134,6 +2447,11 @@ static void launch_d(const AttnArgs& a, const Plan& p, int q_dtype, bool rowmask
   if (p.mfma) {
     if (q_dtype == KVQ_BF16) launch_mfma<D, KVQ_BF16>(a, p.rows, rowmask, grid, st);
     else launch_mfma<D, KVQ_F16>(a, p.rows, rowmask, grid, st);
+    return;
+  }
+  if (p.f32_block) {
+    if (a.bt) hipLaunchKernelGGL((decode_attn_f32_block_kernel<D, true>), grid, dim3(64 * kBlockWaves), 0, st, a);
+    else hipLaunchKernelGGL((decode_attn_f32_block_kernel<D, false>), grid, dim3(64 * kBlockWaves), 0, st, a);
     return;
   }
   switch (q_dtype) {
@@ -2388,6 +2706,9 @@ static int decode_attn_impl(const void* q, int q_dtype, const int64_t* q_strides
   // 16-byte q loads need unit element stride and 16-byte aligned rows.
   a.q_vec = (q_dtype != KVQ_F32 && q_strides[3] == 1 && (uintptr_t)q % 16 == 0 &&
              q_strides[0] % 8 == 0 && q_strides[1] % 8 == 0 && q_strides[2] % 8 == 0) ? 1 : 0;
+  if (q_dtype == KVQ_F32)  // (the block kernel's) 16-byte loads of four fp32 elements
+    a.q_vec = (q_strides[3] == 1 && (uintptr_t)q % 16 == 0 && q_strides[0] % 4 == 0 && q_strides[1] % 4 == 0 &&
+               q_strides[2] % 4 == 0) ? 1 : 0;
   {
     // 4-element output stores: unit dim stride, every row start a multiple of
     // 4 elements, a base aligned to 4 elements (D is a multiple of 4)
