@@ -84,6 +84,23 @@ int kvq_quantize(const void* x, int x_dtype, const int64_t* x_strides,
                  void* stream);
 
 /*
+ * kvq_quantize_kv — kvq_quantize of a layer's K and V in one launch: two
+ * tensors of one shape, dtype, scale dtype and destination rows (capacity,
+ * positions), each with its own pointers and strides. The same bytes as two
+ * kvq_quantize calls (which the reference makes, models/llama3/kv_cache.py:76-102).
+ */
+int kvq_quantize_kv(const void* k, const int64_t* k_strides,
+                    const void* v, const int64_t* v_strides,
+                    int x_dtype, int64_t B, int64_t H, int64_t S, int64_t D, int64_t group_size,
+                    void* k_packed, const int64_t* kp_strides,
+                    void* k_scales, const int64_t* ks_strides,
+                    void* v_packed, const int64_t* vp_strides,
+                    void* v_scales, const int64_t* vs_strides,
+                    int scale_dtype,
+                    const int32_t* write_pos, int64_t write_pos0, int64_t capacity,
+                    void* stream);
+
+/*
  * kvq_dequantize — unpack + scale back to floating point.
  *
  * Replaces kernels/llama3/quantize.py:274-308 dequantize_int4 (CPU semantics
@@ -310,6 +327,20 @@ int kvq_quantize_paged(const void* x, int x_dtype, const int64_t* x_strides,
                        int64_t num_blocks, int64_t page_size,
                        const int32_t* write_pos, int64_t write_pos0,
                        void* stream);
+
+/* kvq_quantize_kv through a block table (both pools' strides are (head, row)). */
+int kvq_quantize_kv_paged(const void* k, const int64_t* k_strides,
+                          const void* v, const int64_t* v_strides,
+                          int x_dtype, int64_t B, int64_t H, int64_t S, int64_t D, int64_t group_size,
+                          void* k_pool, const int64_t* kp_strides,
+                          void* k_scale_pool, const int64_t* ks_strides,
+                          void* v_pool, const int64_t* vp_strides,
+                          void* v_scale_pool, const int64_t* vs_strides,
+                          int scale_dtype,
+                          const int32_t* block_table, int64_t table_stride, int64_t table_cols,
+                          int64_t num_blocks, int64_t page_size,
+                          const int32_t* write_pos, int64_t write_pos0,
+                          void* stream);
 
 int kvq_dequantize_paged(const void* packed_pool, const int64_t* pool_strides,
                          const void* scale_pool, int scale_dtype, const int64_t* scale_pool_strides,

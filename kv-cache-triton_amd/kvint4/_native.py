@@ -31,6 +31,7 @@ EXPORTED_SYMBOLS = (
     "kvq_version",
     "kvq_last_error",
     "kvq_quantize",
+    "kvq_quantize_kv",
     "kvq_dequantize",
     "kvq_decode_attn_num_splits",
     "kvq_decode_attn_workspace_bytes",
@@ -38,6 +39,7 @@ EXPORTED_SYMBOLS = (
     "kvq_decode_step",
     "kvq_decode_step_noalloc",
     "kvq_quantize_paged",
+    "kvq_quantize_kv_paged",
     "kvq_dequantize_paged",
     "kvq_decode_attn_paged",
     "kvq_decode_step_paged",
@@ -69,6 +71,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.kvq_quantize.argtypes = [
         _vp, _i32, _i64p, _i64, _i64, _i64, _i64, _i64,
         _vp, _i64p, _vp, _i32, _i64p, _vp, _i64, _i64, _vp,
+    ]
+    lib.kvq_quantize_kv.restype = _i32
+    lib.kvq_quantize_kv.argtypes = [
+        _vp, _i64p, _vp, _i64p, _i32, _i64, _i64, _i64, _i64, _i64,
+        _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _i32, _vp, _i64, _i64, _vp,
     ]
     lib.kvq_dequantize.restype = _i32
     lib.kvq_dequantize.argtypes = [
@@ -140,6 +147,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.kvq_quantize_paged.argtypes = [
         _vp, _i32, _i64p, _i64, _i64, _i64, _i64, _i64,
         _vp, _i64p, _vp, _i32, _i64p, *pg, _vp, _i64, _vp,
+    ]
+    lib.kvq_quantize_kv_paged.restype = _i32
+    lib.kvq_quantize_kv_paged.argtypes = [
+        _vp, _i64p, _vp, _i64p, _i32, _i64, _i64, _i64, _i64, _i64,
+        _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _i32, *pg, _vp, _i64, _vp,
     ]
     lib.kvq_dequantize_paged.restype = _i32
     lib.kvq_dequantize_paged.argtypes = [

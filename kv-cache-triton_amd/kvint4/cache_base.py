@@ -201,8 +201,8 @@ class QuantizedKVCacheBase:
         start = 0 if prev is None else prev.seq_len
         layer = self._ensure_layer(key_states, layer_idx, start + S)
         pos = layer.seq_lens if layer.seq_lens is not None else start
-        ops.quantize_into(key_states, layer.k_packed, layer.k_scales, self.group_size, pos)
-        ops.quantize_into(value_states, layer.v_packed, layer.v_scales, self.group_size, pos)
+        ops.quantize_kv_into(key_states, value_states, layer.k_packed, layer.k_scales, layer.v_packed, layer.v_scales,
+                             self.group_size, pos)
         if layer.seq_lens is not None:
             layer.seq_lens.add_(S)
         layer.seq_len = start + S

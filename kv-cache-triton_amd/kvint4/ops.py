@@ -100,6 +100,23 @@ def quantize_into(
     cache's capacity raise ValueError) or a device int32 tensor [B] of
     per-sequence positions (rows past the capacity are dropped).
     """
+    wp_ptr, wp0, write_pos = _check_quantize_into(x, packed, scales, group_size, write_pos)
+    B, H, S, D = x.shape
+    lib = nat.lib()
+    with nat.device_of(x):
+        rc = lib.kvq_quantize(
+            x.data_ptr(), nat.DTYPE_CODE[x.dtype], nat.i64_array(x.stride()),
+            B, H, S, D, group_size,
+            packed.data_ptr(), nat.i64_array(packed.stride()[:3]),
+            scales.data_ptr(), nat.DTYPE_CODE[scales.dtype], nat.i64_array(scales.stride()[:3]),
+            wp_ptr, wp0, min(int(packed.shape[2]), int(scales.shape[2])), nat.stream_handle(x.device),
+        )
+    nat.check(rc, "kvq_quantize")
+
+
+def _check_quantize_into(x, packed, scales, group_size, write_pos) -> tuple:
+    """Argument checks of quantize_into: (position pointer or None, scalar
+    position, the tensor behind the pointer)."""
     _check_cuda(x, packed, scales, what="quantize_into")
     if x.dim() != 4 or packed.dim() != 4 or scales.dim() != 4:
         raise ValueError("quantize_into expects 4D x, packed and scales")
@@ -122,16 +139,43 @@ def quantize_into(
         wp0 = int(write_pos)
         if wp0 < 0 or wp0 + S > packed.shape[2] or wp0 + S > scales.shape[2]:
             raise ValueError("write position out of the cache's range")
+    return wp_ptr, wp0, write_pos
+
+
+def quantize_kv_into(
+    k: torch.Tensor,
+    v: torch.Tensor,
+    k_packed: torch.Tensor,
+    k_scales: torch.Tensor,
+    v_packed: torch.Tensor,
+    v_scales: torch.Tensor,
+    group_size: int,
+    write_pos: int | torch.Tensor = 0,
+) -> None:
+    """quantize_into of a layer's K and V [B, H, S, D] in one launch: the
+    same bytes as two calls. Tensors that do not pair (different shapes,
+    dtypes or devices, or none on a GPU) take two."""
+    cap = min(k_packed.shape[2], k_scales.shape[2]) if k_packed.dim() == 4 and k_scales.dim() == 4 else -1
+    if (not k.is_cuda or k.shape != v.shape or k.dtype != v.dtype or k.device != v.device
+            or k_scales.dtype != v_scales.dtype or v_packed.dim() != 4 or v_scales.dim() != 4 or min(v_packed.shape[2], v_scales.shape[2]) != cap):
+        quantize_into(k, k_packed, k_scales, group_size, write_pos)
+        quantize_into(v, v_packed, v_scales, group_size, write_pos)
+        return
+    wp_ptr, wp0, write_pos = _check_quantize_into(k, k_packed, k_scales, group_size, write_pos)
+    _check_quantize_into(v, v_packed, v_scales, group_size, write_pos)
+    B, H, S, D = k.shape
     lib = nat.lib()
-    with nat.device_of(x):
-        rc = lib.kvq_quantize(
-            x.data_ptr(), nat.DTYPE_CODE[x.dtype], nat.i64_array(x.stride()),
-            B, H, S, D, group_size,
-            packed.data_ptr(), nat.i64_array(packed.stride()[:3]),
-            scales.data_ptr(), nat.DTYPE_CODE[scales.dtype], nat.i64_array(scales.stride()[:3]),
-            wp_ptr, wp0, min(int(packed.shape[2]), int(scales.shape[2])), nat.stream_handle(x.device),
+    with nat.device_of(k):
+        rc = lib.kvq_quantize_kv(
+            k.data_ptr(), nat.i64_array(k.stride()), v.data_ptr(), nat.i64_array(v.stride()),
+            nat.DTYPE_CODE[k.dtype], B, H, S, D, group_size,
+            k_packed.data_ptr(), nat.i64_array(k_packed.stride()[:3]),
+            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:3]),
+            v_packed.data_ptr(), nat.i64_array(v_packed.stride()[:3]),
+            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:3]),
+            nat.DTYPE_CODE[k_scales.dtype], wp_ptr, wp0, cap, nat.stream_handle(k.device),
         )
-    nat.check(rc, "kvq_quantize")
+    nat.check(rc, "kvq_quantize_kv")
 
 
 def quantize(x: torch.Tensor, group_size: int, scale_dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
@@ -718,6 +762,21 @@ def quantize_into_paged(
     """quantize_into for a paged cache: row (b, h, s) of x [B, H, S, D] goes to
     sequence b's position pos_b + s, i.e. its page's pool row; positions whose
     page has no block are dropped."""
+    wp_ptr, wp0, write_pos = _check_quantize_into_paged(x, pool, scales, pt, group_size, write_pos)
+    B, H, S, D = x.shape
+    lib = nat.lib()
+    with nat.device_of(x):
+        rc = lib.kvq_quantize_paged(
+            x.data_ptr(), nat.DTYPE_CODE[x.dtype], nat.i64_array(x.stride()),
+            B, H, S, D, group_size,
+            pool.data_ptr(), nat.i64_array(pool.stride()[:2]),
+            scales.data_ptr(), nat.DTYPE_CODE[scales.dtype], nat.i64_array(scales.stride()[:2]),
+            *pt.args(), wp_ptr, wp0, nat.stream_handle(x.device),
+        )
+    nat.check(rc, "kvq_quantize_paged")
+
+
+def _check_quantize_into_paged(x, pool, scales, pt, group_size, write_pos) -> tuple:
     _check_cuda(x, pool, scales, pt.table, what="quantize_into_paged")
     if x.dim() != 4:
         raise ValueError("quantize_into_paged expects 4D x")
@@ -735,16 +794,41 @@ def quantize_into_paged(
         wp0 = int(write_pos)
         if wp0 < 0:
             raise ValueError("write position must be >= 0")
+    return wp_ptr, wp0, write_pos
+
+
+def quantize_kv_into_paged(
+    k: torch.Tensor,
+    v: torch.Tensor,
+    k_pool: torch.Tensor,
+    k_scales: torch.Tensor,
+    v_pool: torch.Tensor,
+    v_scales: torch.Tensor,
+    pt: PageTable,
+    group_size: int,
+    write_pos: int | torch.Tensor = 0,
+) -> None:
+    """quantize_kv_into for a paged cache."""
+    if (not k.is_cuda or k.shape != v.shape or k.dtype != v.dtype or k.device != v.device
+            or k_scales.dtype != v_scales.dtype):
+        quantize_into_paged(k, k_pool, k_scales, pt, group_size, write_pos)
+        quantize_into_paged(v, v_pool, v_scales, pt, group_size, write_pos)
+        return
+    wp_ptr, wp0, write_pos = _check_quantize_into_paged(k, k_pool, k_scales, pt, group_size, write_pos)
+    _check_quantize_into_paged(v, v_pool, v_scales, pt, group_size, write_pos)
+    B, H, S, D = k.shape
     lib = nat.lib()
-    with nat.device_of(x):
-        rc = lib.kvq_quantize_paged(
-            x.data_ptr(), nat.DTYPE_CODE[x.dtype], nat.i64_array(x.stride()),
-            B, H, S, D, group_size,
-            pool.data_ptr(), nat.i64_array(pool.stride()[:2]),
-            scales.data_ptr(), nat.DTYPE_CODE[scales.dtype], nat.i64_array(scales.stride()[:2]),
-            *pt.args(), wp_ptr, wp0, nat.stream_handle(x.device),
+    with nat.device_of(k):
+        rc = lib.kvq_quantize_kv_paged(
+            k.data_ptr(), nat.i64_array(k.stride()), v.data_ptr(), nat.i64_array(v.stride()),
+            nat.DTYPE_CODE[k.dtype], B, H, S, D, group_size,
+            k_pool.data_ptr(), nat.i64_array(k_pool.stride()[:2]),
+            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:2]),
+            v_pool.data_ptr(), nat.i64_array(v_pool.stride()[:2]),
+            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:2]),
+            nat.DTYPE_CODE[k_scales.dtype], *pt.args(), wp_ptr, wp0, nat.stream_handle(k.device),
         )
-    nat.check(rc, "kvq_quantize_paged")
+    nat.check(rc, "kvq_quantize_kv_paged")
 
 
 def dequantize_paged(

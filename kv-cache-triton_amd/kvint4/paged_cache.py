@@ -236,8 +236,7 @@ class PagedQuantizedKVCache:
         pools = self._pools[layer_idx]
         pt = self._page_table()
         pos = self._seq_lens[layer_idx]
-        ops.quantize_into_paged(key_states, pools[0], pools[1], pt, self.group_size, pos)
-        ops.quantize_into_paged(value_states, pools[2], pools[3], pt, self.group_size, pos)
+        ops.quantize_kv_into_paged(key_states, value_states, *pools, pt, self.group_size, pos)
         pos.add_(S)
         self._lens[layer_idx] = [n + S for n in lens]
 
@@ -260,8 +259,7 @@ class PagedQuantizedKVCache:
         pt = self._page_table()
         # rows past a sequence's length land in its last page's slack or, past
         # its pages, are dropped by the kernel; either way they are never read
-        ops.quantize_into_paged(key_states, pools[0], pools[1], pt, self.group_size, 0)
-        ops.quantize_into_paged(value_states, pools[2], pools[3], pt, self.group_size, 0)
+        ops.quantize_kv_into_paged(key_states, value_states, *pools, pt, self.group_size, 0)
         self._lens[layer_idx] = lens
         self._seq_lens[layer_idx].copy_(torch.tensor(lens, dtype=torch.int32))
 
