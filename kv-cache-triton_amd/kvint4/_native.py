@@ -1,4 +1,6 @@
-"""ctypes binding of libkvint4.so (the C ABI declared in include/kvint4.h).
+"""Binding of libkvint4.so (the C ABI declared in include/kvint4.h): through
+the CPython module ``_kvq_host`` (csrc/kvq_pyhost.c) for the operators, which
+pass it tensors, and through ctypes for everything else.
 
 The shared library is built in-tree by ``kvint4.build`` (hipcc, gfx950). There
 is deliberately no fallback: if the library is missing every operator raises,
@@ -15,6 +17,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libkvint4.so")
+HOST_PATH = os.path.join(_HERE, "_kvq_host.so")
 
 KVQ_BF16, KVQ_F16, KVQ_F32 = 0, 1, 2
 KVQ_OK, KVQ_EINVAL, KVQ_ESPACE, KVQ_EHIP, KVQ_EUNSUP = 0, -1, -2, -3, -4
@@ -51,6 +54,7 @@ EXPORTED_SYMBOLS = (
 
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 _i64 = ctypes.c_int64
 _i32 = ctypes.c_int
@@ -205,6 +209,21 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def host():
+    """The CPython module over the native library (built beside it); raises
+    if it was never built."""
+    global _host
+    if _host is None:
+        lib()  # its presence and version are checked there
+        try:
+            from . import _kvq_host
+        except ImportError as e:
+            raise RuntimeError(f"kvint4: {HOST_PATH} cannot be loaded ({e}); build it first "
+                               "(python -m kvint4.build, or __graft_entry__.build())") from e
+        _host = _kvq_host
+    return _host
+
+
 def last_error() -> str:
     msg = lib().kvq_last_error()
     return msg.decode("utf-8", "replace") if msg else ""
@@ -228,22 +247,29 @@ def i64_array(values) -> ctypes.Array:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The handle of torch's current stream of `device`."""
+    idx = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx)
 
 
 class device_of:
-    """Make `tensor`'s device current for the duration of a native call."""
+    """Make `tensor`'s device current for the duration of a native call; the
+    context's value is the handle of the device's current stream."""
+
+    __slots__ = ("idx", "prev")
 
     def __init__(self, t: torch.Tensor):
-        self.idx = t.device.index
+        self.idx = t.get_device()
+        if self.idx < 0:
+            raise ValueError(f"expected a GPU tensor (got one on {t.device})")
         self.prev = None
 
-    def __enter__(self):
-        cur = torch.cuda.current_device()
-        if self.idx is not None and cur != self.idx:
+    def __enter__(self) -> int:
+        cur = torch._C._cuda_getDevice()
+        if cur != self.idx:
             self.prev = cur
             torch.cuda.set_device(self.idx)
-        return self
+        return torch._C._cuda_getCurrentRawStream(self.idx)
 
     def __exit__(self, *exc):
         if self.prev is not None:

@@ -112,9 +112,35 @@ def _build_libs(libs, verbose: bool) -> None:
         shutil.rmtree(tmpdir, ignore_errors=True)
 
 
+# The CPython module that calls the product library with arguments taken from
+# tensors: plain C against the library (found beside it at run time).
+HOST_SRC = os.path.join(CSRC, "kvq_pyhost.c")
+HOST_OUT = os.path.join(_HERE, "_kvq_host.so")
+
+
+def _build_host(verbose: bool) -> None:
+    import sysconfig
+
+    tmpdir = tempfile.mkdtemp(prefix="kvint4-build.", dir=_HERE)
+    try:
+        tmp = os.path.join(tmpdir, os.path.basename(HOST_OUT))
+        cmd = [os.environ.get("CC") or "gcc", "-O2", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"], HOST_SRC,
+               "-o", tmp, "-L" + _HERE, "-l:" + os.path.basename(OUT), "-Wl,-rpath,$ORIGIN"]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"host module build failed ({proc.returncode}):\n{proc.stdout}\n{proc.stderr}")
+        os.replace(tmp, HOST_OUT)
+    finally:
+        shutil.rmtree(tmpdir, ignore_errors=True)
+
+
 def build(verbose: bool = False) -> str:
     """Compile every HIP source into kvint4/libkvint4.so (the product) and
-    kvint4/libkvq_probe.so (measurement only); return the product's path."""
+    kvint4/libkvq_probe.so (measurement only), and the CPython module over the
+    product, kvint4/_kvq_host.so; return the product's path."""
     _build_libs([(OUT, [(s, SOURCE_FLAGS.get(s, ())) for s in SOURCES]), (PROBE_OUT, list(PROBE_SOURCES))],
                 verbose)
+    _build_host(verbose)
     return OUT

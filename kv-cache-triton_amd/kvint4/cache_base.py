@@ -281,8 +281,8 @@ class QuantizedKVCacheBase:
         if layer is None:
             raise KeyError(f"no cache state for layer {layer_idx}")
         n = layer.seq_len
-        return (layer.k_packed[:, :, :n], layer.k_scales[:, :, :n],
-                layer.v_packed[:, :, :n], layer.v_scales[:, :, :n])
+        return (layer.k_packed.narrow(2, 0, n), layer.k_scales.narrow(2, 0, n),
+                layer.v_packed.narrow(2, 0, n), layer.v_scales.narrow(2, 0, n))
 
     def _dequantized(self, layer_idx: int, out_dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
         kp, ks, vp, vs = self.get_quantized(layer_idx)

@@ -102,14 +102,10 @@ def quantize_into(
     """
     wp_ptr, wp0, write_pos = _check_quantize_into(x, packed, scales, group_size, write_pos)
     B, H, S, D = x.shape
-    lib = nat.lib()
-    with nat.device_of(x):
-        rc = lib.kvq_quantize(
-            x.data_ptr(), nat.DTYPE_CODE[x.dtype], nat.i64_array(x.stride()),
-            B, H, S, D, group_size,
-            packed.data_ptr(), nat.i64_array(packed.stride()[:3]),
-            scales.data_ptr(), nat.DTYPE_CODE[scales.dtype], nat.i64_array(scales.stride()[:3]),
-            wp_ptr, wp0, min(int(packed.shape[2]), int(scales.shape[2])), nat.stream_handle(x.device),
+    with nat.device_of(x) as stream:
+        rc = nat.host().quantize(
+            x, nat.DTYPE_CODE[x.dtype], B, H, S, D, group_size, packed, scales, nat.DTYPE_CODE[scales.dtype],
+            wp_ptr, wp0, min(packed.shape[2], scales.shape[2]), stream,
         )
     nat.check(rc, "kvq_quantize")
 
@@ -164,16 +160,10 @@ def quantize_kv_into(
     wp_ptr, wp0, write_pos = _check_quantize_into(k, k_packed, k_scales, group_size, write_pos)
     _check_quantize_into(v, v_packed, v_scales, group_size, write_pos)
     B, H, S, D = k.shape
-    lib = nat.lib()
-    with nat.device_of(k):
-        rc = lib.kvq_quantize_kv(
-            k.data_ptr(), nat.i64_array(k.stride()), v.data_ptr(), nat.i64_array(v.stride()),
-            nat.DTYPE_CODE[k.dtype], B, H, S, D, group_size,
-            k_packed.data_ptr(), nat.i64_array(k_packed.stride()[:3]),
-            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:3]),
-            v_packed.data_ptr(), nat.i64_array(v_packed.stride()[:3]),
-            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:3]),
-            nat.DTYPE_CODE[k_scales.dtype], wp_ptr, wp0, cap, nat.stream_handle(k.device),
+    with nat.device_of(k) as stream:
+        rc = nat.host().quantize_kv(
+            k, v, nat.DTYPE_CODE[k.dtype], B, H, S, D, group_size, k_packed, k_scales, v_packed, v_scales,
+            nat.DTYPE_CODE[k_scales.dtype], wp_ptr, wp0, cap, stream,
         )
     nat.check(rc, "kvq_quantize_kv")
 
@@ -191,14 +181,11 @@ def quantize(x: torch.Tensor, group_size: int, scale_dtype: torch.dtype) -> tupl
     xv, sizes, strides = _as_bhs(x)
     pv = packed.reshape(*sizes, w)
     sv = scales.reshape(*sizes, ng)
-    lib = nat.lib()
-    with nat.device_of(x):
-        rc = lib.kvq_quantize(
-            xv.data_ptr(), nat.DTYPE_CODE[x.dtype], nat.i64_array((*strides, xv.stride(-1))),
-            sizes[0], sizes[1], sizes[2], d, group_size,
-            pv.data_ptr(), nat.i64_array(pv.stride()[:3]),
-            sv.data_ptr(), nat.DTYPE_CODE[scale_dtype], nat.i64_array(sv.stride()[:3]),
-            None, 0, sizes[2], nat.stream_handle(x.device),
+    with nat.device_of(x) as stream:
+        rc = nat.host().quantize(
+            (xv.data_ptr(), (*strides, xv.stride(-1))), nat.DTYPE_CODE[x.dtype],
+            sizes[0], sizes[1], sizes[2], d, group_size, pv, sv, nat.DTYPE_CODE[scale_dtype],
+            None, 0, sizes[2], stream,
         )
     nat.check(rc, "kvq_quantize")
     return packed, scales
@@ -232,14 +219,10 @@ def dequantize(
         sv = scales.reshape(*sizes, ng)
         sstr = sv.stride()[:3]
     ov = out.reshape(*sizes, d_out)
-    lib = nat.lib()
-    with nat.device_of(packed):
-        rc = lib.kvq_dequantize(
-            pv.data_ptr(), nat.i64_array(pstr),
-            sv.data_ptr(), nat.DTYPE_CODE[scales.dtype], nat.i64_array(sstr),
-            sizes[0], sizes[1], sizes[2], group_size, ng,
-            ov.data_ptr(), nat.DTYPE_CODE[out_dtype], nat.i64_array(ov.stride()), d_out,
-            nat.stream_handle(packed.device),
+    with nat.device_of(packed) as stream:
+        rc = nat.host().dequantize(
+            (pv.data_ptr(), pstr), (sv.data_ptr(), sstr), nat.DTYPE_CODE[scales.dtype],
+            sizes[0], sizes[1], sizes[2], group_size, ng, ov, nat.DTYPE_CODE[out_dtype], d_out, stream,
         )
     nat.check(rc, "kvq_dequantize")
     return out
@@ -355,6 +338,27 @@ def _num_cus(device: torch.device) -> int:
     return n
 
 
+def _plan(q: torch.Tensor, B: int, Hq: int, n_kv_heads: int, Sq: int, D: int, s_max: int,
+          qd: int, sd: int, n_split: int | None) -> tuple[int, int]:
+    """(splits, workspace bytes) of a decode launch."""
+    if n_split is not None and n_split < 1:
+        raise ValueError("n_split must be >= 1")
+    n, ws_bytes = nat.host().plan(B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, _num_cus(q.device), n_split or 0)
+    if n < 0:
+        nat.check(n, "kvq_decode_attn_num_splits")
+    if ws_bytes < 0:
+        nat.check(ws_bytes, "kvq_decode_attn_workspace_bytes")
+    return n, ws_bytes
+
+
+def _decode_ws(q: torch.Tensor, stream: int, ws_bytes: int) -> tuple:
+    """(pointer, bytes) of the split workspace of a launch on `stream`."""
+    if ws_bytes <= 0:
+        return None, 0
+    ws = _workspaces.get(q.device, stream, ws_bytes)
+    return ws.data_ptr(), ws.numel()
+
+
 def fused_decode_attention(
     q: torch.Tensor,
     k_packed: torch.Tensor,
@@ -392,35 +396,14 @@ def fused_decode_attention(
             raise ValueError("seq_lens must be a device int32 tensor of shape [B]")
         seq_lens = seq_lens.contiguous()
         sl_ptr = seq_lens.data_ptr()
-    lib = nat.lib()
     qd = nat.DTYPE_CODE[q.dtype]
     sd = nat.DTYPE_CODE[k_scales.dtype]
-    if n_split is None:
-        n_split = lib.kvq_decode_attn_num_splits(B, Hq, n_kv_heads, Sq, D, Sk, qd, sd, _num_cus(q.device))
-        if n_split < 0:
-            nat.check(int(n_split), "kvq_decode_attn_num_splits")
-    elif n_split < 1:
-        raise ValueError("n_split must be >= 1")
-    ws_bytes = lib.kvq_decode_attn_workspace_bytes(B, Hq, n_kv_heads, Sq, D, qd, sd, n_split)
-    if ws_bytes < 0:
-        nat.check(int(ws_bytes), "kvq_decode_attn_workspace_bytes")
-    with nat.device_of(q):
-        stream = nat.stream_handle(q.device)
-        ws_ptr, ws_len = None, 0
-        if ws_bytes > 0:
-            ws = _workspaces.get(q.device, stream, ws_bytes)
-            ws_ptr, ws_len = ws.data_ptr(), ws.numel()
-        rc = lib.kvq_decode_attn(
-            q.data_ptr(), qd, nat.i64_array(q.stride()),
-            k_packed.data_ptr(), nat.i64_array(k_packed.stride()[:3]),
-            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:3]),
-            v_packed.data_ptr(), nat.i64_array(v_packed.stride()[:3]),
-            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:3]),
-            sd,
-            out.data_ptr(), nat.i64_array(out.stride()),
-            B, Hq, n_kv_heads, Sq, D, group_size, Sk,
-            sl_ptr, 1 if is_causal else 0, float(sm_scale),
-            n_split, ws_ptr, ws_len, stream,
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, Sk, qd, sd, n_split)
+    with nat.device_of(q) as stream:
+        ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
+        rc = nat.host().decode_attn(
+            q, qd, k_packed, k_scales, v_packed, v_scales, sd, out, B, Hq, n_kv_heads, Sq, D, group_size, Sk,
+            sl_ptr, 1 if is_causal else 0, float(sm_scale), n_split, ws_ptr, ws_len, stream,
         )
     nat.check(rc, "kvq_decode_attn")
     return out
@@ -457,20 +440,11 @@ def prefill_attention(
         v_scales = v_scales.contiguous()
     if v_scales.dtype != k_scales.dtype:
         v_scales = v_scales.to(k_scales.dtype)
-    lib = nat.lib()
-    with nat.device_of(q):
-        stream = nat.stream_handle(q.device)
+    with nat.device_of(q) as stream:
         ws, ws_ptr, ws_len = _prefill_ws(q, n_kv_heads, Sk)
-        rc = lib.kvq_prefill_attn(
-            q.data_ptr(), nat.DTYPE_CODE[q.dtype], nat.i64_array(q.stride()),
-            k_packed.data_ptr(), nat.i64_array(k_packed.stride()[:3]),
-            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:3]),
-            v_packed.data_ptr(), nat.i64_array(v_packed.stride()[:3]),
-            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:3]),
-            nat.DTYPE_CODE[k_scales.dtype],
-            out.data_ptr(), nat.i64_array(out.stride()),
-            B, Hq, n_kv_heads, Sq, D, group_size, Sk,
-            1 if is_causal else 0, float(sm_scale), ws_ptr, ws_len, stream,
+        rc = nat.host().prefill_attn(
+            q, nat.DTYPE_CODE[q.dtype], k_packed, k_scales, v_packed, v_scales, nat.DTYPE_CODE[k_scales.dtype], out,
+            B, Hq, n_kv_heads, Sq, D, group_size, Sk, 1 if is_causal else 0, float(sm_scale), ws_ptr, ws_len, stream,
         )
     nat.check(rc, "kvq_prefill_attn")
     return out
@@ -511,44 +485,24 @@ def decode_step(
         k_new = k_new.contiguous()
     if v_new.stride(-1) != 1:
         v_new = v_new.contiguous()
-    lib = nat.lib()
     qd = nat.DTYPE_CODE[q.dtype]
     sd = nat.DTYPE_CODE[k_scales.dtype]
     if isinstance(position, torch.Tensor):
         if position.dtype != torch.int32 or not position.is_cuda or position.numel() != B:
             raise ValueError("position must be an int or a device int32 tensor of shape [B]")
-        pos_ptr, pos0, s_max = position.contiguous().data_ptr(), 0, cap
+        position = position.contiguous()
+        pos_ptr, pos0, s_max = position.data_ptr(), 0, cap
     else:
         pos_ptr, pos0 = None, int(position)
         if not 0 <= pos0 < cap:
             raise ValueError(f"write position {pos0} outside the cache capacity {cap}")
         s_max = pos0 + 1
-    if n_split is None:
-        n_split = lib.kvq_decode_attn_num_splits(B, Hq, n_kv_heads, 1, D, s_max, qd, sd, _num_cus(q.device))
-        if n_split < 0:
-            nat.check(int(n_split), "kvq_decode_attn_num_splits")
-    ws_bytes = lib.kvq_decode_attn_workspace_bytes(B, Hq, n_kv_heads, 1, D, qd, sd, n_split)
-    if ws_bytes < 0:
-        nat.check(int(ws_bytes), "kvq_decode_attn_workspace_bytes")
-    with nat.device_of(q):
-        stream = nat.stream_handle(q.device)
-        ws_ptr, ws_len = None, 0
-        if ws_bytes > 0:
-            ws = _workspaces.get(q.device, stream, ws_bytes)
-            ws_ptr, ws_len = ws.data_ptr(), ws.numel()
-        rc = lib.kvq_decode_step(
-            q.data_ptr(), qd, nat.i64_array(q.stride()),
-            k_new.data_ptr(), nat.i64_array(k_new.stride()),
-            v_new.data_ptr(), nat.i64_array(v_new.stride()),
-            k_packed.data_ptr(), nat.i64_array(k_packed.stride()[:3]),
-            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:3]),
-            v_packed.data_ptr(), nat.i64_array(v_packed.stride()[:3]),
-            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:3]),
-            sd,
-            out.data_ptr(), nat.i64_array(out.stride()),
-            B, Hq, n_kv_heads, D, group_size, cap,
-            pos_ptr, pos0, float(sm_scale),
-            n_split, ws_ptr, ws_len, stream,
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, 1, D, s_max, qd, sd, n_split)
+    with nat.device_of(q) as stream:
+        ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
+        rc = nat.host().decode_step(
+            q, qd, k_new, v_new, k_packed, k_scales, v_packed, v_scales, sd, out, B, Hq, n_kv_heads, D, group_size,
+            cap, pos_ptr, pos0, float(sm_scale), n_split, ws_ptr, ws_len, stream,
         )
     nat.check(rc, "kvq_decode_step")
     return out
@@ -764,14 +718,10 @@ def quantize_into_paged(
     page has no block are dropped."""
     wp_ptr, wp0, write_pos = _check_quantize_into_paged(x, pool, scales, pt, group_size, write_pos)
     B, H, S, D = x.shape
-    lib = nat.lib()
-    with nat.device_of(x):
-        rc = lib.kvq_quantize_paged(
-            x.data_ptr(), nat.DTYPE_CODE[x.dtype], nat.i64_array(x.stride()),
-            B, H, S, D, group_size,
-            pool.data_ptr(), nat.i64_array(pool.stride()[:2]),
-            scales.data_ptr(), nat.DTYPE_CODE[scales.dtype], nat.i64_array(scales.stride()[:2]),
-            *pt.args(), wp_ptr, wp0, nat.stream_handle(x.device),
+    with nat.device_of(x) as stream:
+        rc = nat.host().quantize_paged(
+            x, nat.DTYPE_CODE[x.dtype], B, H, S, D, group_size, pool, scales, nat.DTYPE_CODE[scales.dtype],
+            pt.args(), wp_ptr, wp0, stream,
         )
     nat.check(rc, "kvq_quantize_paged")
 
@@ -817,16 +767,10 @@ def quantize_kv_into_paged(
     wp_ptr, wp0, write_pos = _check_quantize_into_paged(k, k_pool, k_scales, pt, group_size, write_pos)
     _check_quantize_into_paged(v, v_pool, v_scales, pt, group_size, write_pos)
     B, H, S, D = k.shape
-    lib = nat.lib()
-    with nat.device_of(k):
-        rc = lib.kvq_quantize_kv_paged(
-            k.data_ptr(), nat.i64_array(k.stride()), v.data_ptr(), nat.i64_array(v.stride()),
-            nat.DTYPE_CODE[k.dtype], B, H, S, D, group_size,
-            k_pool.data_ptr(), nat.i64_array(k_pool.stride()[:2]),
-            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:2]),
-            v_pool.data_ptr(), nat.i64_array(v_pool.stride()[:2]),
-            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:2]),
-            nat.DTYPE_CODE[k_scales.dtype], *pt.args(), wp_ptr, wp0, nat.stream_handle(k.device),
+    with nat.device_of(k) as stream:
+        rc = nat.host().quantize_kv_paged(
+            k, v, nat.DTYPE_CODE[k.dtype], B, H, S, D, group_size, k_pool, k_scales, v_pool, v_scales,
+            nat.DTYPE_CODE[k_scales.dtype], pt.args(), wp_ptr, wp0, stream,
         )
     nat.check(rc, "kvq_quantize_kv_paged")
 
@@ -851,32 +795,13 @@ def dequantize_paged(
     out = torch.empty((B, H, S, d_out), dtype=out_dtype, device=pool.device)
     if out.numel() == 0:
         return out
-    lib = nat.lib()
-    with nat.device_of(pool):
-        rc = lib.kvq_dequantize_paged(
-            pool.data_ptr(), nat.i64_array(pool.stride()[:2]),
-            scales.data_ptr(), nat.DTYPE_CODE[scales.dtype], nat.i64_array(scales.stride()[:2]),
-            *pt.args(), B, H, S, group_size, ng,
-            out.data_ptr(), nat.DTYPE_CODE[out_dtype], nat.i64_array(out.stride()), d_out,
-            nat.stream_handle(pool.device),
+    with nat.device_of(pool) as stream:
+        rc = nat.host().dequantize_paged(
+            pool, scales, nat.DTYPE_CODE[scales.dtype], pt.args(), B, H, S, group_size, ng, out,
+            nat.DTYPE_CODE[out_dtype], d_out, stream,
         )
     nat.check(rc, "kvq_dequantize_paged")
     return out
-
-
-def _plan(lib, q: torch.Tensor, B: int, Hq: int, n_kv_heads: int, Sq: int, D: int, s_max: int,
-          sd: int, n_split: int | None) -> tuple[int, int]:
-    qd = nat.DTYPE_CODE[q.dtype]
-    if n_split is None:
-        n_split = lib.kvq_decode_attn_num_splits(B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, _num_cus(q.device))
-        if n_split < 0:
-            nat.check(int(n_split), "kvq_decode_attn_num_splits")
-    elif n_split < 1:
-        raise ValueError("n_split must be >= 1")
-    ws_bytes = lib.kvq_decode_attn_workspace_bytes(B, Hq, n_kv_heads, Sq, D, qd, sd, n_split)
-    if ws_bytes < 0:
-        nat.check(int(ws_bytes), "kvq_decode_attn_workspace_bytes")
-    return int(n_split), int(ws_bytes)
 
 
 def fused_decode_attention_paged(
@@ -922,26 +847,13 @@ def fused_decode_attention_paged(
             raise ValueError(f"seq_len must be in [0, {pt.capacity}] when seq_lens is not given")
         seq_len = int(seq_len)
         s_max = seq_len
-    lib = nat.lib()
-    sd = nat.DTYPE_CODE[k_scales.dtype]
-    n_split, ws_bytes = _plan(lib, q, B, Hq, n_kv_heads, Sq, D, s_max, sd, n_split)
-    with nat.device_of(q):
-        stream = nat.stream_handle(q.device)
-        ws_ptr, ws_len = None, 0
-        if ws_bytes > 0:
-            ws = _workspaces.get(q.device, stream, ws_bytes)
-            ws_ptr, ws_len = ws.data_ptr(), ws.numel()
-        rc = lib.kvq_decode_attn_paged(
-            q.data_ptr(), nat.DTYPE_CODE[q.dtype], nat.i64_array(q.stride()),
-            k_pool.data_ptr(), nat.i64_array(k_pool.stride()[:2]),
-            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:2]),
-            v_pool.data_ptr(), nat.i64_array(v_pool.stride()[:2]),
-            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:2]),
-            sd, *pt.args(),
-            out.data_ptr(), nat.i64_array(out.stride()),
-            B, Hq, n_kv_heads, Sq, D, group_size,
-            sl_ptr, seq_len, 1 if is_causal else 0, float(sm_scale),
-            n_split, ws_ptr, ws_len, stream,
+    qd, sd = nat.DTYPE_CODE[q.dtype], nat.DTYPE_CODE[k_scales.dtype]
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, n_split)
+    with nat.device_of(q) as stream:
+        ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
+        rc = nat.host().decode_attn_paged(
+            q, qd, k_pool, k_scales, v_pool, v_scales, sd, pt.args(), out, B, Hq, n_kv_heads, Sq, D, group_size,
+            sl_ptr, seq_len, 1 if is_causal else 0, float(sm_scale), n_split, ws_ptr, ws_len, stream,
         )
     nat.check(rc, "kvq_decode_attn_paged")
     return out
@@ -979,20 +891,12 @@ def prefill_attention_paged(
         out = torch.empty_like(q)
     if v_scales.dtype != k_scales.dtype:
         raise nat.KVQUnsupported("K and V scales must share a dtype")
-    lib = nat.lib()
-    with nat.device_of(q):
-        stream = nat.stream_handle(q.device)
+    with nat.device_of(q) as stream:
         ws, ws_ptr, ws_len = _prefill_ws(q, n_kv_heads, seq_len)
-        rc = lib.kvq_prefill_attn_paged(
-            q.data_ptr(), nat.DTYPE_CODE[q.dtype], nat.i64_array(q.stride()),
-            k_pool.data_ptr(), nat.i64_array(k_pool.stride()[:2]),
-            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:2]),
-            v_pool.data_ptr(), nat.i64_array(v_pool.stride()[:2]),
-            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:2]),
-            nat.DTYPE_CODE[k_scales.dtype], *pt.args(),
-            out.data_ptr(), nat.i64_array(out.stride()),
-            B, Hq, n_kv_heads, Sq, D, group_size, seq_len,
-            1 if is_causal else 0, float(sm_scale), ws_ptr, ws_len, stream,
+        rc = nat.host().prefill_attn_paged(
+            q, nat.DTYPE_CODE[q.dtype], k_pool, k_scales, v_pool, v_scales, nat.DTYPE_CODE[k_scales.dtype], pt.args(),
+            out, B, Hq, n_kv_heads, Sq, D, group_size, seq_len, 1 if is_causal else 0, float(sm_scale), ws_ptr, ws_len,
+            stream,
         )
     nat.check(rc, "kvq_prefill_attn_paged")
     return out
@@ -1038,34 +942,20 @@ def decode_step_paged(
     if isinstance(position, torch.Tensor):
         if position.dtype != torch.int32 or not position.is_cuda or position.numel() != B:
             raise ValueError("position must be an int or a device int32 tensor of shape [B]")
-        pos_ptr, pos0, s_max = position.contiguous().data_ptr(), 0, cap
+        position = position.contiguous()
+        pos_ptr, pos0, s_max = position.data_ptr(), 0, cap
     else:
         pos_ptr, pos0 = None, int(position)
         if not 0 <= pos0 < cap:
             raise ValueError(f"write position {pos0} outside the table's capacity {cap}")
         s_max = pos0 + 1
-    lib = nat.lib()
-    sd = nat.DTYPE_CODE[k_scales.dtype]
-    n_split, ws_bytes = _plan(lib, q, B, Hq, n_kv_heads, 1, D, s_max, sd, n_split)
-    with nat.device_of(q):
-        stream = nat.stream_handle(q.device)
-        ws_ptr, ws_len = None, 0
-        if ws_bytes > 0:
-            ws = _workspaces.get(q.device, stream, ws_bytes)
-            ws_ptr, ws_len = ws.data_ptr(), ws.numel()
-        rc = lib.kvq_decode_step_paged(
-            q.data_ptr(), nat.DTYPE_CODE[q.dtype], nat.i64_array(q.stride()),
-            k_new.data_ptr(), nat.i64_array(k_new.stride()),
-            v_new.data_ptr(), nat.i64_array(v_new.stride()),
-            k_pool.data_ptr(), nat.i64_array(k_pool.stride()[:2]),
-            k_scales.data_ptr(), nat.i64_array(k_scales.stride()[:2]),
-            v_pool.data_ptr(), nat.i64_array(v_pool.stride()[:2]),
-            v_scales.data_ptr(), nat.i64_array(v_scales.stride()[:2]),
-            sd, *pt.args(),
-            out.data_ptr(), nat.i64_array(out.stride()),
-            B, Hq, n_kv_heads, D, group_size,
-            pos_ptr, pos0, float(sm_scale),
-            n_split, ws_ptr, ws_len, stream,
+    qd, sd = nat.DTYPE_CODE[q.dtype], nat.DTYPE_CODE[k_scales.dtype]
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, 1, D, s_max, qd, sd, n_split)
+    with nat.device_of(q) as stream:
+        ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
+        rc = nat.host().decode_step_paged(
+            q, qd, k_new, v_new, k_pool, k_scales, v_pool, v_scales, sd, pt.args(), out, B, Hq, n_kv_heads, D,
+            group_size, pos_ptr, pos0, float(sm_scale), n_split, ws_ptr, ws_len, stream,
         )
     nat.check(rc, "kvq_decode_step_paged")
     return out
