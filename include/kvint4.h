@@ -145,6 +145,24 @@ int64_t kvq_decode_attn_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int6
                                         int64_t n_split);
 
 /*
+ * Splits by length: n_split = KVQ_SPLIT_BY_LENGTH in kvq_decode_attn,
+ * kvq_decode_step and their paged forms, with per-sequence device lengths
+ * (seq_lens / positions) and a workspace of at least
+ * kvq_decode_attn_by_length_workspace_bytes(...) bytes: the splits are dealt to
+ * the sequences by their lengths, on the device, so that a batch of very
+ * different lengths keeps the device busy. The figure is 0 where the plan of
+ * kvq_decode_attn_num_splits is to be used instead (bf16/fp16 with D = 128, one
+ * query position and 2 to 64 sequences are supported; short caches gain
+ * nothing), and never more than kvq_decode_attn_workspace_bytes of 64 splits.
+ * In any other call a large n_split means as many equal splits as the cap
+ * allows, as before.
+ */
+#define KVQ_SPLIT_BY_LENGTH (1 << 30)
+int64_t kvq_decode_attn_by_length_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
+                                                  int64_t D, int64_t s_max, int q_dtype,
+                                                  int scale_dtype);
+
+/*
  * kvq_decode_attn — fused INT4 GQA attention for short query blocks (decode).
  *
  * Replaces kernels/llama3/attention_quant.py:159-286 attention_forward_quant_gqa

@@ -129,6 +129,9 @@ struct AttnArgs {
   int64_t bt_stride;
   int bt_cols, n_blocks, page_shift;
   uint32_t pool_rows;
+  // splits by length (kernels instantiated with RAGGED): work items per
+  // (KV head, row chunk), workgroups of a round among them, sequences
+  int items, slots, batch;
   uint32_t* ws_cnt;  // [kCntUnits] arrival counters, kCntStride words apart
                      // (zero between calls)
   float* ws_ml;      // [n_units][n_split][ROWS][2]  (max, sum)
@@ -221,6 +224,10 @@ __device__ __forceinline__ void permlane16_swap(float& x, float& y) {
   y = __builtin_bit_cast(float, r1);
 }
 
+__device__ __forceinline__ float readlane_f(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+
 // Full-wave reductions; the result is read from lane 63 and is wave-uniform.
 __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, dpp<0x111>(v, kNeg));  // row_shr:1
@@ -273,6 +280,105 @@ __device__ __forceinline__ void unit_coords(const AttnArgs& a, int unit, int& b,
   rc = unit - (int)bh * a.row_chunks;
   b = (int)fdiv(bh, a.div_hkv);
   kvh = (int)bh - b * a.Hkv;
+}
+
+// Wave-wide helpers on integers (every lane active).
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+#define KVQ_SCAN_STEP(ctrl, mask) v += __builtin_amdgcn_update_dpp(0, v, ctrl, mask, 0xF, false)
+  KVQ_SCAN_STEP(0x111, 0xF);  // row_shr:1, 2, 4, 8
+  KVQ_SCAN_STEP(0x112, 0xF);
+  KVQ_SCAN_STEP(0x114, 0xF);
+  KVQ_SCAN_STEP(0x118, 0xF);
+  KVQ_SCAN_STEP(0x142, 0xA);  // row_bcast:15, 31
+  KVQ_SCAN_STEP(0x143, 0xC);
+#undef KVQ_SCAN_STEP
+  return v;
+}
+__device__ __forceinline__ float wave_sum_lane63(float v) {
+  v += dpp<0x111>(v, 0.0f);
+  v += dpp<0x112>(v, 0.0f);
+  v += dpp<0x114>(v, 0.0f);
+  v += dpp<0x118>(v, 0.0f);
+  v += dpp<0x142, 0xA>(v, 0.0f);
+  v += dpp<0x143, 0xC>(v, 0.0f);
+  return v;
+}
+// ceil(n / w) for 0 <= n <= 2^26, 64 <= w <= 2^26 with inv ~ 1 / w: the float
+// quotient is within one of it.
+__device__ __forceinline__ int ceil_div(int n, int w, float inv) {
+  int q = (int)((float)n * inv);
+  q += q * w < n ? 1 : 0;
+  q += q * w < n ? 1 : 0;
+  q -= q > 0 && (q - 1) * w >= n ? 1 : 0;
+  return q;
+}
+
+// Splits by length: a batch of very different lengths (device lengths, at
+// most 64 sequences, one per lane). With one split count for all, the longest
+// sequence's workgroups outlast the rest (a paged batch of 32 sequences of 256
+// to 16K keys, one split each: 66 us, of which the bytes need 28; 38 us by length). Here every split holds W
+// keys, sequence b has ns_b = max(1, ceil(L_b / W)) of them, and the launch's
+// workgroups are items of one list per (KV head, row chunk): sequence 0's
+// splits, sequence 1's, ... Every wave works the list out from the lengths,
+// lane b holding sequence b's.
+// W = the longest length / k, for the k of a table whose estimate is the
+// shortest: with all items in one round of resident workgroups W + A keys,
+// else the average (T + A items) / slots plus half of that; A = 1200 keys
+// stands for a workgroup's prologue, fold and merge. The estimates count items
+// in floats; if the exact count of the chosen W does not fit the list, W is
+// the longest length (one item per sequence, which the host leaves room for).
+// Item -> (b, split, ns, first item of b, W); false: no such item.
+__device__ __forceinline__ bool ragged_item(const AttnArgs& a, int item, int& b, int& split, int& ns, int& first,
+                                            int& W_out, int& len_b) {
+  const int lane = threadIdx.x & 63;
+  const bool seq = lane < a.batch;
+  const int raw = seq ? a.seq_lens[lane] : 0;
+  const int len = raw < 0 ? 0 : (raw < a.Sk ? raw : a.Sk);
+  const float lenf = (float)len;
+  const float T = readlane_f(wave_sum_lane63(lenf), 63);
+  const float mx = wave_max(lenf);
+  const float slots = (float)a.slots, inv_slots = 1.0f / slots, items = (float)a.items;
+  const int w1 = max(((int)mx + 63) & ~63, 256);
+  constexpr int NC = 12;
+  constexpr float K[NC] = {1.0f, 2.0f, 3.0f, 4.0f, 5.0f, 6.0f, 8.0f, 10.0f, 12.0f, 16.0f, 24.0f, 32.0f};
+  int Wc[NC];
+  float cnt[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    Wc[c] = max(((int)(mx * (1.0f / K[c]) + 0.999f) + 63) & ~63, 256);
+    const float n = fmaxf(ceilf(lenf * __builtin_amdgcn_rcpf((float)Wc[c])), 1.0f);
+    cnt[c] = seq ? n : 0.0f;
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) cnt[c] = readlane_f(wave_sum_lane63(cnt[c]), 63);
+  const float A = 1200.0f;
+  float best = 3.0e38f;
+  int W = w1;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const float w = (float)Wc[c];
+    const float cost = cnt[c] <= slots ? w + A : (T + A * cnt[c]) * inv_slots + 0.5f * (w + A);
+    const bool take = cost < best && cnt[c] <= items;
+    best = take ? cost : best;
+    W = take ? Wc[c] : W;
+  }
+  W = __builtin_amdgcn_readfirstlane(W);
+  int n = seq ? max(ceil_div(len, W, 1.0f / (float)W), 1) : 0;
+  int incl = wave_inclusive_sum(n);
+  if (__builtin_amdgcn_readlane(incl, 63) > a.items) {
+    W = w1;
+    n = seq ? 1 : 0;
+    incl = wave_inclusive_sum(n);
+  }
+  if (item >= __builtin_amdgcn_readlane(incl, 63)) return false;
+  b = (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(seq && incl <= item));
+  b = __builtin_amdgcn_readfirstlane(b);
+  ns = __builtin_amdgcn_readlane(n, b);
+  first = __builtin_amdgcn_readlane(incl, b) - ns;
+  len_b = __builtin_amdgcn_readlane(raw, b);
+  split = item - first;
+  W_out = W;
+  return true;
 }
 
 __device__ __forceinline__ int64_t out_index(const AttnArgs& a, int b, int kvh, int rho, int d) {
@@ -440,7 +546,7 @@ __device__ __forceinline__ float group_reduce(float v) {
 // outputs of their pieces. A row no split saw a key for (all l_s = 0) yields
 // zeros.
 template <int ROWS, int D, int OUT_DT, int NW>
-__device__ __forceinline__ void merge_splits(const AttnArgs& a, int unit, int rc, int kvh, int b,
+__device__ __forceinline__ void merge_splits(const AttnArgs& a, int64_t part0, int ns, int rc, int kvh, int b,
                                              MergeLds& mg) {
   constexpr int NT = 64 * NW;
   constexpr int Q = ROWS * D / 4;  // 16-byte pieces per split
@@ -451,11 +557,10 @@ __device__ __forceinline__ void merge_splits(const AttnArgs& a, int unit, int rc
   constexpr int MLPT = (kMaxSplit * kMaxRows + NT - 1) / NT;  // (max, sum) loads per thread
   constexpr int PW = 64 / P;       // pieces per wave
   const int tid = threadIdx.x;
-  const int ns = a.n_split;
   const int lane = tid & 63;
   const int piece = (tid >> 6) * PW + lane % PW, grp = lane / PW;
   const int r = piece / (D / 4), d4 = piece % (D / 4);
-  const int64_t slot0 = (int64_t)unit * ns * ROWS;  // + split * ROWS + row
+  const int64_t slot0 = part0 * ROWS;  // + split * ROWS + row
   const __amdgpu_buffer_rsrc_t ro =
       buffer_rsrc(a.ws_o + slot0 * D, (uint32_t)((int64_t)ns * ROWS * D * 4));
   const __amdgpu_buffer_rsrc_t rm = buffer_rsrc(a.ws_ml + slot0 * 2, (uint32_t)(ns * ROWS * 8));
@@ -556,14 +661,17 @@ __device__ __forceinline__ void merge_splits(const AttnArgs& a, int unit, int rc
 // waves' ones: its score per row at nt[r] (max = score, sum = 1; kNeg for a
 // row it is masked from) and its values at nt[ROWS + d], the same for every
 // row. The MFMA kernel's decode step passes the new token this way.
+//
+// The unit has ns splits, whose partials are slots part0 .. part0 + ns - 1 of
+// the workspace.
 template <int ROWS, int D, int OUT_DT, int NW>
-__device__ __forceinline__ void finish_block(const AttnArgs& a, int unit, int split, int rc,
+__device__ __forceinline__ void finish_block(const AttnArgs& a, int unit, int split, int ns, int64_t part0, int rc,
                                              int kvh, int b, const float (*o_lds)[ROWS][D],
                                              const float (*ml_lds)[ROWS][2], MergeLds& mg,
                                              const float* nt = nullptr) {
   constexpr int NT = 64 * NW;
   const int tid = threadIdx.x;
-  const bool single = a.n_split == 1;
+  const bool single = ns == 1;
   for (int idx = tid; idx < ROWS * D; idx += NT) {
     const int r = idx / D, d = idx % D;
     float mw[NW], lw[NW];
@@ -594,7 +702,7 @@ __device__ __forceinline__ void finish_block(const AttnArgs& a, int unit, int sp
       if (rho < a.rows_total)
         store_from_f32(a.out, out_index(a, b, kvh, rho, d), OUT_DT, Ls > 0.0f ? Os / Ls : 0.0f);
     } else {
-      const int64_t slot = ((int64_t)unit * a.n_split + split) * ROWS + r;
+      const int64_t slot = (part0 + split) * ROWS + r;
       a.ws_o[slot * D + d] = Os;
       if (d == 0) *(float2*)&a.ws_ml[slot * 2] = make_float2(M, Ls);
     }
@@ -607,12 +715,12 @@ __device__ __forceinline__ void finish_block(const AttnArgs& a, int unit, int sp
   uint32_t* cnt = a.ws_cnt + (int64_t)unit * kCntStride;
   if (tid == 0)
     mg.last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-              (uint32_t)(a.n_split - 1);
+              (uint32_t)(ns - 1);
     KVQ_STAMP(7);
   __syncthreads();
   if (!mg.last) return;
   KVQ_STAMP(8);
-  merge_splits<ROWS, D, OUT_DT, NW>(a, unit, rc, kvh, b, mg);
+  merge_splits<ROWS, D, OUT_DT, NW>(a, part0, ns, rc, kvh, b, mg);
   if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -656,9 +764,6 @@ __device__ __forceinline__ float row16_sum(float m) {
       "v_add_f32_dpp %0, %0, %0 row_ror:1 row_mask:0xf bank_mask:0xf"
       : "+v"(m));
   return m;
-}
-__device__ __forceinline__ float readlane_f(float v, int lane) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
 template <bool SUM>
 __device__ __forceinline__ void wave_reduce4(const float x[4], float out[4]) {
@@ -705,7 +810,8 @@ __device__ __forceinline__ void chunk_scales(uint2 raw, bool g32, const uint32_t
 template <int D, int RS>
 constexpr int mfma_waves_per_simd() { return D == 64 && RS == 1 ? 4 : (RS == 2 ? 2 : 1); }
 
-template <int D, int RS, int QM, int SM, bool ROWMASK, int NW, int CH, bool PAGED>
+// RAGGED: the launch's splits are items by length (ragged_item).
+template <int D, int RS, int QM, int SM, bool ROWMASK, int NW, int CH, bool PAGED, bool RAGGED>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd<D, RS>())))
 void decode_attn_mfma_kernel(const AttnArgs a) {
   constexpr bool F16 = QM == KVQ_F16;
@@ -789,8 +895,23 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
   // the query's LDS reads (a scalar load in flight turns those reads' waits
   // into waits for it too).
   asm volatile("" ::"s"(a.bt_cols), "s"(a.ws_o));
-  int unit, split;
-  if (!unit_and_split(a, unit, split)) return;
+  int unit, split, b, kvh, rc;
+  int ns, split_keys = 0, L;  // the unit's splits; (RAGGED) keys of a split; the sequence's length
+  int64_t part0;              // the unit's first partial slot
+  if constexpr (RAGGED) {
+    const int hc = (int)((blockIdx.x & 7u) + 8u * blockIdx.y);
+    int first;
+    if (hc >= a.Hkv * a.row_chunks || !ragged_item(a, (int)(blockIdx.x >> 3), b, split, ns, first, split_keys, L))
+      return;
+    kvh = (int)fdiv((uint32_t)hc, a.div_rc);
+    rc = hc - kvh * a.row_chunks;
+    unit = (b * a.Hkv + kvh) * a.row_chunks + rc;
+    part0 = (int64_t)hc * a.items + first;
+  } else {
+    if (!unit_and_split(a, unit, split)) return;
+    ns = a.n_split;
+    part0 = (int64_t)unit * ns;
+  }
   // The two waves of a SIMD (w and w + 4) run the same scalar prologue, and a
   // SIMD issues one scalar instruction per turn: raising the first one's
   // priority until its first tiles' loads are issued lets it reach them in
@@ -803,15 +924,16 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
   // 9.33 -> 9.26 us, C2 7.27 -> 7.29 us; with four waves per SIMD, C5 lost
   // 0.28 us that way).
   {
-    const bool app = D == 128 && RS == 1 && a.append && split == a.n_split - 1 && (wave % (NW / 2)) >= NW / 2 - 2;
+    const bool app = D == 128 && RS == 1 && a.append && split == ns - 1 && (wave % (NW / 2)) >= NW / 2 - 2;
     if ((wave < NW / 2) != app) __builtin_amdgcn_s_setprio(1);
   }
-  int b, kvh, rc;
-  unit_coords(a, unit, b, kvh, rc);
-  // the sequence's length is read first (its latency then overlaps the query
-  // loads, which do not depend on it)
-  int L = a.append ? a.pos0 : a.Sk;
-  if (a.seq_lens) L = load_const_i32(a.seq_lens, b);
+  if constexpr (!RAGGED) {
+    unit_coords(a, unit, b, kvh, rc);
+    // the sequence's length is read first (its latency then overlaps the query
+    // loads, which do not depend on it)
+    L = a.append ? a.pos0 : a.Sk;
+    if (a.seq_lens) L = load_const_i32(a.seq_lens, b);
+  }
 
   // ---- query rows first (wave-private copy: QT pieces of 8 elements, lane
   //      handles pieces lane, lane + 64, ...; rows past the last one read row
@@ -845,7 +967,7 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
   L = L < 0 ? 0 : L;
   // decode step: the new token goes to row L (if it fits the cache) and is
   // attended by the unit's last split from registers
-  bool has_new = a.append && len_ok && L < a.Sk && split == a.n_split - 1;
+  bool has_new = a.append && len_ok && L < a.Sk && split == ns - 1;
   L = L < a.Sk ? L : a.Sk;
   // The new token's rows (lane l: elements 2l, 2l+1): the K row for the
   // split's last wave, which quantizes, stores and scores it, the V row for
@@ -871,8 +993,14 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
   };
   if constexpr (EARLY_NEW) load_new_row();
   int t_begin, t_end;
-  if constexpr (PAGED) split_range64(a, L, split, t_begin, t_end);
-  else split_range(a, L, split, t_begin, t_end);
+  if constexpr (RAGGED) {
+    t_begin = split * split_keys;
+    t_end = min(L, t_begin + split_keys);
+  } else if constexpr (PAGED) {
+    split_range64(a, L, split, t_begin, t_end);
+  } else {
+    split_range(a, L, split, t_begin, t_end);
+  }
   const int32_t* bt_b = PAGED ? a.bt + (int64_t)b * a.bt_stride : nullptr;
   // paged: the block of this wave's first tile, read here so that the table
   // read's latency overlaps the rest of the prologue (read where the tile's
@@ -1573,7 +1701,7 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
   __syncthreads();
   // the new token (scores and values in LDS, written by the K and V waves
   // before their tile loops) joins the waves' partials in the workgroup fold
-  finish_block<ROWS, D, QM, NW>(a, unit, split, rc, kvh, b, o_lds, ml_lds, mg, has_new ? nt_lds : nullptr);
+  finish_block<ROWS, D, QM, NW>(a, unit, split, ns, part0, rc, kvh, b, o_lds, ml_lds, mg, has_new ? nt_lds : nullptr);
   KVQ_STAMP(11);
 }
 
@@ -2276,7 +2404,8 @@ __global__ __launch_bounds__(256) void decode_attn_valu_kernel(const AttnArgs a)
   __syncthreads();
   // the new token (scores and values in LDS, written by waves 3 and 2 before
   // their tile loops) joins the waves' partials in the workgroup fold
-  finish_block<ROWS, D, QM, 4>(a, unit, split, rc, kvh, b, o_lds, ml_lds, mg, has_new ? nt_lds : nullptr);
+  finish_block<ROWS, D, QM, 4>(a, unit, split, a.n_split, (int64_t)unit * a.n_split, rc, kvh, b, o_lds, ml_lds, mg,
+                               has_new ? nt_lds : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -2380,6 +2509,37 @@ static int64_t workspace_bytes_for(const Plan& p, int64_t D) {
   return ws_cnt_bytes(p) + ws_ml_bytes(p) + (int64_t)p.n_units * p.n_split * p.rows * D * 4;
 }
 
+// Splits by length (RAGGED kernels): D = 128, one query position, matching
+// 16-bit types, 2 to 64 sequences. Items per (KV head, row chunk): one round
+// of workgroups (a CU holds one) for up to 5/8 as many sequences, two for up
+// to 3/2, a round more than the sequences need beyond. Workgroups whose item
+// does not exist exit after working out the list, but in a launch of more than
+// one round they do that behind the others (about 2 us), so rounds are not
+// added freely. The partials are slots of the items, so the
+// workspace does not depend on the lengths; it is never more than a plan of
+// kMaxSplit equal splits needs.
+struct RaggedPlan {
+  int items, slots;  // items = 0: not for this shape
+  int64_t bytes;
+};
+
+static RaggedPlan ragged_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t D, int q_dtype, int scale_dtype) {
+  RaggedPlan r = {0, 0, 0};
+  if (D != 128 || Sq != 1 || B < 2 || B > 64 || q_dtype != scale_dtype || q_dtype == KVQ_F32) return r;
+  Plan p;
+  if (make_plan(B, Hq, Hkv, Sq, D, 1, q_dtype, scale_dtype, 1, 1, &p) != KVQ_OK || p.n_units > kCntUnits) return r;
+  const int64_t hc = p.n_units / B;
+  const int64_t slots = (256 + hc - 1) / hc;
+  const int64_t items = (8 * B <= 5 * slots ? 1 : (2 * B <= 3 * slots ? 2 : 1 + (B + slots - 1) / slots)) * slots;
+  if (items > kMaxSplit * B) return r;
+  p.n_units = (int)hc;
+  p.n_split = (int)items;
+  r.items = (int)items;
+  r.slots = (int)slots;
+  r.bytes = workspace_bytes_for(p, D);
+  return r;
+}
+
 // Waves per workgroup of the MFMA kernel: 8 (two per SIMD hide each other's
 // latency), with one tile's loads in flight per wave (the SIMD partner covers
 // the latency; a second slot measured 5-12 % slower from 4K to 128K keys with
@@ -2395,8 +2555,14 @@ template <int D, int RS, int QM, int SM, bool PAGED>
 static void launch_mfma_rs(const AttnArgs& a, bool rowmask, dim3 grid, hipStream_t st) {
   constexpr int NW = mfma_waves<RS>();
   constexpr int CH = mfma_tiles_in_flight<RS>();
-  if (rowmask) hipLaunchKernelGGL((decode_attn_mfma_kernel<D, RS, QM, SM, true, NW, CH, PAGED>), grid, dim3(64 * NW), 0, st, a);
-  else hipLaunchKernelGGL((decode_attn_mfma_kernel<D, RS, QM, SM, false, NW, CH, PAGED>), grid, dim3(64 * NW), 0, st, a);
+  if constexpr (D == 128 && QM == SM) {
+    if (a.items > 0) {
+      hipLaunchKernelGGL((decode_attn_mfma_kernel<D, RS, QM, SM, false, NW, CH, PAGED, true>), grid, dim3(64 * NW), 0, st, a);
+      return;
+    }
+  }
+  if (rowmask) hipLaunchKernelGGL((decode_attn_mfma_kernel<D, RS, QM, SM, true, NW, CH, PAGED, false>), grid, dim3(64 * NW), 0, st, a);
+  else hipLaunchKernelGGL((decode_attn_mfma_kernel<D, RS, QM, SM, false, NW, CH, PAGED, false>), grid, dim3(64 * NW), 0, st, a);
 }
 
 template <int D, int QM, bool PAGED>
@@ -2494,6 +2660,27 @@ extern "C" int64_t kvq_decode_attn_num_splits(int64_t B, int64_t Hq, int64_t Hkv
     return rc;
   }
   return p.n_split;
+}
+
+extern "C" int64_t kvq_decode_attn_by_length_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
+                                                             int64_t D, int64_t s_max, int q_dtype,
+                                                             int scale_dtype) {
+  clear_error();
+  if (!dtype_ok(q_dtype) || !dtype_ok(scale_dtype)) {
+    set_error("kvq_decode_attn_by_length_workspace_bytes: q and scale dtypes must be bf16/fp16/fp32");
+    return KVQ_EINVAL;
+  }
+  // Working out the items costs every workgroup a load round trip and about
+  // 300 instructions before its first load (1 to 2 us), which a batch of
+  // unequal lengths wins back from about 64K rows of capacity on (lengths
+  // spread over the logarithm of [cap / 64, cap], GQA 4, equal splits / by
+  // length, us: 2 x 8K 8.9 / 10.4, 8 x 4K 11.0 / 11.1, 8 x 8K 14.9 / 13.0, 4 x
+  // 16K 14.4 / 11.3, 16 x 16K 36.7 / 25.7, 32 x 16K 62 / 36), and where the
+  // items take more than one round, from 8K rows a sequence (32 x 4K 19.9 /
+  // 20.6, 32 x 8K 34 / 28.5).
+  if (s_max < 4096 || B * s_max < 65536) return 0;
+  const RaggedPlan r = ragged_plan(B, Hq, Hkv, Sq, D, q_dtype, scale_dtype);
+  return r.items > r.slots && s_max < 8192 ? 0 : r.bytes;
 }
 
 extern "C" int64_t kvq_decode_attn_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
@@ -2662,13 +2849,19 @@ static int decode_attn_impl(const void* q, int q_dtype, const int64_t* q_strides
     set_error("kvq_decode_attn: unsupported shape");
     return rc;
   }
-  const int64_t need = workspace_bytes_for(p, D);
+  // splits by length, if asked for and the workspace holds them
+  RaggedPlan rag = {0, 0, 0};
+  if (n_split >= KVQ_SPLIT_BY_LENGTH && seq_lens != nullptr && p.mfma) {
+    rag = ragged_plan(B, Hq, Hkv, Sq, D, q_dtype, scale_dtype);
+    if (rag.items > 0 && (workspace == nullptr || workspace_bytes < rag.bytes)) rag.items = 0;
+  }
+  const int64_t need = rag.items > 0 ? rag.bytes : workspace_bytes_for(p, D);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
     set_error("kvq_decode_attn: workspace too small (%lld < %lld bytes)",
               (long long)workspace_bytes, (long long)need);
     return KVQ_ESPACE;
   }
-  if (p.n_split > 1) {
+  if (p.n_split > 1 || rag.items > 0) {
     const int drc = split_merge_device_ok();
     if (drc != KVQ_OK) return drc;
   }
@@ -2737,6 +2930,10 @@ static int decode_attn_impl(const void* q, int q_dtype, const int64_t* q_strides
 #endif
   if (need > 0) {
     char* w = (char*)workspace;
+    if (rag.items > 0) {  // the partials' geometry: items per head chunk
+      p.n_split = rag.items;
+      p.n_units = p.n_units / (int)B;
+    }
     a.ws_cnt = (uint32_t*)w;
     a.ws_ml = (float*)(w + ws_cnt_bytes(p));
     a.ws_o = (float*)(w + ws_cnt_bytes(p) + ws_ml_bytes(p));
@@ -2748,6 +2945,9 @@ static int decode_attn_impl(const void* q, int q_dtype, const int64_t* q_strides
   const int64_t gy = std::min<int64_t>(groups, 32768), gz = (groups + gy - 1) / gy;
   const dim3 grid((unsigned)(8 * p.n_split), (unsigned)gy, (unsigned)gz);
   a.grid_y = (int)gy;
+  a.items = rag.items;
+  a.slots = rag.slots;
+  a.batch = (int)B;
   hipStream_t st = (hipStream_t)stream;
   if (D == 128) launch_d<128>(a, p, q_dtype, rowmask, grid, st);
   else launch_d<64>(a, p, q_dtype, rowmask, grid, st);

@@ -232,12 +232,18 @@ FN(py_dequantize_paged) {
                             s[0], s[1], s[2], s[3], s[4], o.p, (int)d[0], o.st, d[1], st));
 }
 
-/* (B, Hq, Hkv, Sq, D, s_max, q_dtype, scale_dtype, num_cus, n_split or 0) -> (n_split, workspace bytes), either
-   negative: a status of kvq_decode_attn_num_splits or kvq_decode_attn_workspace_bytes */
+/* (B, Hq, Hkv, Sq, D, s_max, q_dtype, scale_dtype, num_cus, n_split or 0, whether the call has device lengths) ->
+   (n_split, workspace bytes), either negative: a status of kvq_decode_attn_num_splits or
+   kvq_decode_attn_workspace_bytes */
 FN(py_plan) {
-  WANT(10);
-  INTS(s, 0, 10);
+  WANT(11);
+  INTS(s, 0, 11);
   int64_t n = s[9], w = 0;
+  if (n < 1 && s[10]) {
+    w = kvq_decode_attn_by_length_workspace_bytes(s[0], s[1], s[2], s[3], s[4], s[5], (int)s[6], (int)s[7]);
+    if (w > 0) return Py_BuildValue("LL", (long long)KVQ_SPLIT_BY_LENGTH, (long long)w);
+    w = 0;
+  }
   if (n < 1) n = kvq_decode_attn_num_splits(s[0], s[1], s[2], s[3], s[4], s[5], (int)s[6], (int)s[7], s[8]);
   if (n > 0) w = kvq_decode_attn_workspace_bytes(s[0], s[1], s[2], s[3], s[4], (int)s[6], (int)s[7], n);
   return Py_BuildValue("LL", (long long)n, (long long)w);

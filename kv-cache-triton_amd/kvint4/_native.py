@@ -38,6 +38,7 @@ EXPORTED_SYMBOLS = (
     "kvq_dequantize",
     "kvq_decode_attn_num_splits",
     "kvq_decode_attn_workspace_bytes",
+    "kvq_decode_attn_by_length_workspace_bytes",
     "kvq_decode_attn",
     "kvq_decode_step",
     "kvq_decode_step_noalloc",
@@ -90,6 +91,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.kvq_decode_attn_num_splits.argtypes = [_i64, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _i64]
     lib.kvq_decode_attn_workspace_bytes.restype = _i64
     lib.kvq_decode_attn_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64, _i64, _i32, _i32, _i64]
+    lib.kvq_decode_attn_by_length_workspace_bytes.restype = _i64
+    lib.kvq_decode_attn_by_length_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64, _i64, _i64, _i32, _i32]
     lib.kvq_decode_attn.restype = _i32
     lib.kvq_decode_attn.argtypes = [
         _vp, _i32, _i64p,

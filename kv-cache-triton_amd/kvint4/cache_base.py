@@ -43,6 +43,7 @@ class _LayerQuantizedKV:
     v_scales: torch.Tensor
     seq_len: int
     seq_lens: Optional[torch.Tensor] = None
+    ragged: bool = False  # the sequences' lengths differ (load_ragged)
 
     @property
     def capacity(self) -> int:
@@ -243,7 +244,7 @@ class QuantizedKVCacheBase:
             out = ops.decode_step(
                 query_states, key_states, value_states,
                 layer.k_packed, layer.k_scales, layer.v_packed, layer.v_scales, pos,
-                n_kv_heads=n_kv_heads, group_size=self.group_size, sm_scale=scale,
+                n_kv_heads=n_kv_heads, group_size=self.group_size, sm_scale=scale, by_length=layer.ragged,
             )
         except _native.KVQUnsupported:
             return None
@@ -270,6 +271,7 @@ class QuantizedKVCacheBase:
         self._append_quantized(key_states, value_states, layer_idx)
         layer = self._layers[layer_idx]
         layer.seq_lens = lengths.to(device=key_states.device, dtype=torch.int32).clone()
+        layer.ragged = True
 
     def get_seq_lens(self, layer_idx: int) -> Optional[torch.Tensor]:
         """Per-sequence lengths of a ragged layer (device int32 [B]) or None."""

@@ -339,11 +339,13 @@ def _num_cus(device: torch.device) -> int:
 
 
 def _plan(q: torch.Tensor, B: int, Hq: int, n_kv_heads: int, Sq: int, D: int, s_max: int,
-          qd: int, sd: int, n_split: int | None) -> tuple[int, int]:
-    """(splits, workspace bytes) of a decode launch."""
+          qd: int, sd: int, n_split: int | None, lengths: bool) -> tuple[int, int]:
+    """(splits, workspace bytes) of a decode launch; `lengths`: it has device
+    lengths, by which the splits may be dealt to the sequences."""
     if n_split is not None and n_split < 1:
         raise ValueError("n_split must be >= 1")
-    n, ws_bytes = nat.host().plan(B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, _num_cus(q.device), n_split or 0)
+    n, ws_bytes = nat.host().plan(B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, _num_cus(q.device), n_split or 0,
+                                   1 if lengths else 0)
     if n < 0:
         nat.check(n, "kvq_decode_attn_num_splits")
     if ws_bytes < 0:
@@ -398,7 +400,7 @@ def fused_decode_attention(
         sl_ptr = seq_lens.data_ptr()
     qd = nat.DTYPE_CODE[q.dtype]
     sd = nat.DTYPE_CODE[k_scales.dtype]
-    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, Sk, qd, sd, n_split)
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, Sk, qd, sd, n_split, sl_ptr is not None)
     with nat.device_of(q) as stream:
         ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
         rc = nat.host().decode_attn(
@@ -465,6 +467,7 @@ def decode_step(
     sm_scale: float,
     out: torch.Tensor | None = None,
     n_split: int | None = None,
+    by_length: bool = True,
 ) -> torch.Tensor:
     """One decode token in one launch: quantize k_new / v_new [B, Hkv, 1, D]
     into row `position` of the capacity buffers (an int for every sequence, or
@@ -472,7 +475,10 @@ def decode_step(
     over the cache including the new row. The buffers are the cache's
     [B, Hkv, capacity, .] tensors, written in place; the caller advances its
     lengths. Raises KVQUnsupported for dtype/group combinations the fused
-    step does not handle (the caller then quantizes and attends separately)."""
+    step does not handle (the caller then quantizes and attends separately).
+    With device positions a batch's splits are dealt to the sequences by their
+    lengths where that pays; `by_length` = False says that the lengths are
+    alike, so that every sequence gets the same splits without working that out."""
     B, Hq, Sq, D = q.shape
     if Sq != 1:
         raise nat.KVQUnsupported("decode_step handles one query position")
@@ -497,7 +503,7 @@ def decode_step(
         if not 0 <= pos0 < cap:
             raise ValueError(f"write position {pos0} outside the cache capacity {cap}")
         s_max = pos0 + 1
-    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, 1, D, s_max, qd, sd, n_split)
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, 1, D, s_max, qd, sd, n_split, by_length and pos_ptr is not None)
     with nat.device_of(q) as stream:
         ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
         rc = nat.host().decode_step(
@@ -848,7 +854,7 @@ def fused_decode_attention_paged(
         seq_len = int(seq_len)
         s_max = seq_len
     qd, sd = nat.DTYPE_CODE[q.dtype], nat.DTYPE_CODE[k_scales.dtype]
-    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, n_split)
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, n_split, sl_ptr is not None)
     with nat.device_of(q) as stream:
         ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
         rc = nat.host().decode_attn_paged(
@@ -918,10 +924,12 @@ def decode_step_paged(
     sm_scale: float,
     out: torch.Tensor | None = None,
     n_split: int | None = None,
+    by_length: bool = True,
 ) -> torch.Tensor:
     """decode_step over a paged cache: the new token of sequence b goes to its
     position (int, or device int32 [B] of old lengths) through the block table;
-    a position whose page has no block is neither written nor attended."""
+    a position whose page has no block is neither written nor attended.
+    `by_length` as for decode_step."""
     _check_cuda(q, k_new, v_new, k_pool, pt.table, what="decode_step_paged")
     B, Hq, Sq, D = q.shape
     if pt.table.shape[0] < B:
@@ -950,7 +958,7 @@ def decode_step_paged(
             raise ValueError(f"write position {pos0} outside the table's capacity {cap}")
         s_max = pos0 + 1
     qd, sd = nat.DTYPE_CODE[q.dtype], nat.DTYPE_CODE[k_scales.dtype]
-    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, 1, D, s_max, qd, sd, n_split)
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, 1, D, s_max, qd, sd, n_split, by_length and pos_ptr is not None)
     with nat.device_of(q) as stream:
         ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
         rc = nat.host().decode_step_paged(

@@ -284,7 +284,8 @@ class PagedQuantizedKVCache:
         pos = self._seq_lens[layer_idx]
         try:
             out = ops.decode_step_paged(query_states, key_states, value_states, *pools, pt, pos,
-                                        n_kv_heads=n_kv_heads, group_size=self.group_size, sm_scale=scale)
+                                        n_kv_heads=n_kv_heads, group_size=self.group_size, sm_scale=scale,
+                                        by_length=any(n != lens[0] for n in lens))
         except _native.KVQUnsupported:
             return None
         pos.add_(1)

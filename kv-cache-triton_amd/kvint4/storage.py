@@ -118,5 +118,5 @@ def load_cache(path: str, cache: Cache, device: Union[str, torch.device] = "cuda
             continue
         S = parts[0].shape[2]
         ragged = bool((lens != S).any())
-        cache._layers[i] = _LayerQuantizedKV(*parts, S, lens.to(dev) if ragged else None)
+        cache._layers[i] = _LayerQuantizedKV(*parts, S, lens.to(dev) if ragged else None, ragged)
     return cache

@@ -49,6 +49,6 @@ def test_plan_equals_the_planning_functions(shape):
     for qd, sd in ((0, 0), (1, 1), (2, 1)):
         n = lib.kvq_decode_attn_num_splits(*shape, qd, sd, 256)
         w = lib.kvq_decode_attn_workspace_bytes(*shape[:5], qd, sd, n)
-        assert nat.host().plan(*shape, qd, sd, 256, 0) == (n, w)
-        assert nat.host().plan(*shape, qd, sd, 256, 3)[0] == 3
-    assert nat.host().plan(1, 3, 2, 1, 128, 10, 0, 0, 256, 0)[0] == nat.KVQ_EINVAL
+        assert nat.host().plan(*shape, qd, sd, 256, 0, 0) == (n, w)
+        assert nat.host().plan(*shape, qd, sd, 256, 3, 0)[0] == 3
+    assert nat.host().plan(1, 3, 2, 1, 128, 10, 0, 0, 256, 0, 0)[0] == nat.KVQ_EINVAL
