@@ -171,11 +171,15 @@ __device__ __attribute__((noinline)) void store_tile_direct(uint16_t* k_dst, uin
 // RB = 16-row blocks per wave (1 or 2): with two, every K and V fragment read
 // from LDS feeds two MFMAs, halving LDS traffic and dequantize work per row.
 // Two row blocks per wave must stay within 256 registers (two waves per
-// SIMD): one more register halves the occupancy.
-template <int D, bool F16, bool S_F16, int RB, bool PAGED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RB == 2 ? 2 : 1)))
+// SIMD): one more register halves the occupancy. NW = waves per workgroup
+// (4, or 8 for D = 128 with two row blocks): the workgroup's threads share
+// the dequantize of each K/V tile, so eight waves (one workgroup per CU
+// instead of two of four) halve its VALU per wave. Long blocks come here only
+// where they are not staged (no workspace for it, or a head's images over
+// kStageBytes).
+template <int D, bool F16, bool S_F16, int RB, bool PAGED, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(RB == 2 ? 2 : 1)))
 void prefill_attn_kernel(const PrefillArgs a) {
-  constexpr int NW = 4;  // waves per workgroup
   constexpr int NT = 64 * NW;
   constexpr int ROWS = kWaveRows * NW * RB;  // query rows per workgroup
   constexpr int KP = D + 8;      // K tile row pitch in LDS (elements)
@@ -1014,15 +1018,15 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs a,
   store4(a.out + (int64_t)b * a.os_b + (int64_t)head * a.os_h + (int64_t)s * a.os_s + d, w0, w1, a.o_vec);
 }
 
-template <int D, bool F16, int RB>
+template <int D, bool F16, int RB, int NW>
 void launch_prefill(const PrefillArgs& a, bool s_f16, dim3 grid, hipStream_t st) {
-  const dim3 block(256);
+  const dim3 block(64 * NW);
   if (a.bt) {
-    if (s_f16) hipLaunchKernelGGL((prefill_attn_kernel<D, F16, true, RB, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((prefill_attn_kernel<D, F16, false, RB, true>), grid, block, 0, st, a);
+    if (s_f16) hipLaunchKernelGGL((prefill_attn_kernel<D, F16, true, RB, true, NW>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((prefill_attn_kernel<D, F16, false, RB, true, NW>), grid, block, 0, st, a);
   } else {
-    if (s_f16) hipLaunchKernelGGL((prefill_attn_kernel<D, F16, true, RB, false>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((prefill_attn_kernel<D, F16, false, RB, false>), grid, block, 0, st, a);
+    if (s_f16) hipLaunchKernelGGL((prefill_attn_kernel<D, F16, true, RB, false, NW>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((prefill_attn_kernel<D, F16, false, RB, false, NW>), grid, block, 0, st, a);
   }
 }
 
@@ -1033,9 +1037,12 @@ void launch_merge(const PrefillArgs& a, int rows, hipStream_t st) {
 }
 
 template <int D, bool F16>
-void launch_prefill_rb(const PrefillArgs& a, bool s_f16, int rb, dim3 grid, hipStream_t st) {
-  if (rb == 2) launch_prefill<D, F16, 2>(a, s_f16, grid, st);
-  else launch_prefill<D, F16, 1>(a, s_f16, grid, st);
+void launch_prefill_rb(const PrefillArgs& a, bool s_f16, int rb, int nw, dim3 grid, hipStream_t st) {
+  if constexpr (D == 128) {
+    if (nw == 8) return launch_prefill<D, F16, 2, 8>(a, s_f16, grid, st);  // never split
+  }
+  if (rb == 2) launch_prefill<D, F16, 2, 4>(a, s_f16, grid, st);
+  else launch_prefill<D, F16, 1, 4>(a, s_f16, grid, st);
   if (a.n_split > 1) launch_merge<D, F16>(a, kWaveRows * 4 * rb, st);
 }
 
@@ -1054,9 +1061,11 @@ void launch_staged(const PrefillArgs& a, bool s_f16, int nw, hipStream_t st) {
   if (a.n_split > 1) launch_merge<D, F16>(a, 32 * nw, st);
 }
 
-// Launch plan of the unstaged kernel: rows per workgroup (four waves of rb
+// Launch plan of the unstaged kernel: rows per workgroup (nw waves of rb
 // 16-row blocks), row blocks, and the split over keys. Two row blocks per
-// wave once that still gives a workgroup per CU of a 256-CU device. A launch
+// wave once that still gives a workgroup of four waves per CU of a 256-CU
+// device; at D = 128 eight waves once that gives a workgroup per CU (the 16K
+// prompt 2.37 ms, 2.55 with four). A launch
 // of fewer workgroups splits the keys. A tile takes a lone workgroup of a CU
 // about 1.3 us, and two workgroups of a CU together longer, so the target is
 // one workgroup per CU with splits of at least two tiles (D = 128, 8 KV heads,
@@ -1065,20 +1074,21 @@ void launch_staged(const PrefillArgs& a, bool s_f16, int nw, hipStream_t st) {
 // leaves splits of over 1024 keys the launch is long enough to fill 512
 // workgroup slots (two per CU) instead.
 struct PrefillPlan {
-  int rb, n_split;
+  int rb, nw, n_split;
   int64_t row_blocks;
 };
 
-PrefillPlan prefill_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk) {
+PrefillPlan prefill_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D) {
   const int64_t ratio = Hq / Hkv;
   const int64_t rows = Sq * ratio;
   PrefillPlan p;
   p.rb = B * Hkv * ((rows + 8 * kWaveRows - 1) / (8 * kWaveRows)) >= 256 ? 2 : 1;
-  const int64_t wg_rows = kWaveRows * 4 * p.rb;
+  p.nw = D == 128 && p.rb == 2 && B * Hkv * ((rows + 16 * kWaveRows - 1) / (16 * kWaveRows)) >= 256 ? 8 : 4;
+  const int64_t wg_rows = kWaveRows * p.nw * p.rb;
   p.row_blocks = (rows + wg_rows - 1) / wg_rows;
   const int64_t n_wg = B * Hkv * p.row_blocks;
   int64_t ns = 1;
-  if (n_wg > 0 && n_wg < 512) {
+  if (p.nw == 4 && n_wg > 0 && n_wg < 512) {
     ns = std::min<int64_t>((256 + n_wg - 1) / n_wg, std::max<int64_t>(1, Sk / 128));
     if (Sk > 1024 * ns) ns = std::min<int64_t>((512 + n_wg - 1) / n_wg, std::max<int64_t>(1, Sk / 512));
     ns = std::min<int64_t>(ns, 64);
@@ -1089,7 +1099,7 @@ PrefillPlan prefill_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t
 
 int64_t prefill_ws_bytes(const PrefillPlan& p, int64_t B, int64_t Hkv, int64_t D) {
   if (p.n_split <= 1) return 0;
-  return B * Hkv * p.row_blocks * p.n_split * (kWaveRows * 4 * p.rb) * (D + 2) * 4;
+  return B * Hkv * p.row_blocks * p.n_split * (kWaveRows * p.nw * p.rb) * (D + 2) * 4;
 }
 
 // Plan of the staged route. Units go in groups whose images fit kStageBytes
@@ -1211,7 +1221,7 @@ int prefill_impl(const void* q, int q_dtype, const int64_t* q_strides, const voi
   // enough of it the launch is unstaged, then unsplit
   StagedPlan sp = staged_plan(B, Hq, Hkv, Sq, pg && pg->bt_cols == 0 ? 0 : Sk, D);
   if (workspace == nullptr || workspace_bytes < staged_ws_bytes(sp, D) || (uintptr_t)workspace % 16 != 0) sp.nw = 0;
-  PrefillPlan plan = prefill_plan(B, Hq, Hkv, Sq, Sk);
+  PrefillPlan plan = prefill_plan(B, Hq, Hkv, Sq, Sk, D);
   const int64_t need = prefill_ws_bytes(plan, B, Hkv, D);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) plan.n_split = 1;
   const int rb = plan.rb;
@@ -1278,15 +1288,15 @@ int prefill_impl(const void* q, int q_dtype, const int64_t* q_strides, const voi
   }
   a.n_split = plan.n_split;
   a.ws_o = plan.n_split > 1 ? (float*)workspace : nullptr;
-  a.ws_ml = plan.n_split > 1 ? (float*)workspace + B * Hkv * row_blocks * plan.n_split * (kWaveRows * 4 * rb) * D : nullptr;
+  a.ws_ml = plan.n_split > 1 ? (float*)workspace + B * Hkv * row_blocks * plan.n_split * (kWaveRows * plan.nw * rb) * D : nullptr;
 
   const dim3 grid((unsigned)n_wg);
   if (D == 128) {
-    if (f16) launch_prefill_rb<128, true>(a, s_f16, rb, grid, st);
-    else launch_prefill_rb<128, false>(a, s_f16, rb, grid, st);
+    if (f16) launch_prefill_rb<128, true>(a, s_f16, rb, plan.nw, grid, st);
+    else launch_prefill_rb<128, false>(a, s_f16, rb, plan.nw, grid, st);
   } else {
-    if (f16) launch_prefill_rb<64, true>(a, s_f16, rb, grid, st);
-    else launch_prefill_rb<64, false>(a, s_f16, rb, grid, st);
+    if (f16) launch_prefill_rb<64, true>(a, s_f16, rb, plan.nw, grid, st);
+    else launch_prefill_rb<64, false>(a, s_f16, rb, plan.nw, grid, st);
   }
   KVQ_CHECK_LAUNCH("kvq_prefill_attn");
   return KVQ_OK;
@@ -1319,7 +1329,7 @@ extern "C" int64_t kvq_prefill_attn_workspace_bytes(int64_t B, int64_t Hq, int64
     return KVQ_EINVAL;
   }
   if (B == 0 || Sq == 0) return 0;
-  return prefill_ws_bytes(prefill_plan(B, Hq, Hkv, Sq, Sk), B, Hkv, D);
+  return prefill_ws_bytes(prefill_plan(B, Hq, Hkv, Sq, Sk, D), B, Hkv, D);
 }
 
 extern "C" int64_t kvq_prefill_attn_staged_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
