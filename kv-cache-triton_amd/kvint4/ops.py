@@ -32,11 +32,12 @@ MAX_FUSED_ROWS = 1024
 # A block of at least PREFILL_MIN_ROWS rows per KV head whose rows x keys
 # reach PREFILL_MIN_WORK, over a cache with one length for the batch (a
 # prompt, a prompt chunk, a large speculative block), goes to the matrix-core
-# prefill kernel instead: it dequantizes each 64-key tile into LDS once for
-# 64 or 128 rows and splits the key range when the launch is small. Measured
-# crossover with the fused kernel (GQA 4): 64 rows at 16K keys (16 queries
-# 48 vs 60 us), 128-256 at 4K, 512-1024 at 1K; a whole 16K prompt takes
-# 3.50 ms vs 4.50 ms for dequantize + flash SDPA.
+# prefill kernels instead: they dequantize each 64-key tile into LDS once for
+# 64 or 128 rows, or long blocks' keys once for all their rows, and split the
+# key range when the launch is small. Measured crossover with the fused kernel
+# (GQA 4): 64 rows at 16K keys (16 queries 48 vs 60 us), 128-256 at 4K,
+# 512-1024 at 1K; a whole 16K prompt takes 1.9 ms vs 4.5 ms for dequantize +
+# flash SDPA.
 PREFILL_MIN_ROWS = 64
 PREFILL_MIN_WORK = 1 << 20
 
@@ -322,7 +323,14 @@ def _prefill_ws(q: torch.Tensor, Hkv: int, Sk: int) -> tuple:
         nat.check(int(n), "kvq_prefill_attn_staged_workspace_bytes")
     if n == 0:
         return None, None, 0
-    ws = torch.empty(n, dtype=torch.uint8, device=q.device)
+    try:
+        ws = torch.empty(n, dtype=torch.uint8, device=q.device)
+    except torch.cuda.OutOfMemoryError:
+        # a device with less than the images' room left runs unstaged, slower
+        n = nat.lib().kvq_prefill_attn_workspace_bytes(B, Hq, Hkv, Sq, D, Sk)
+        if n <= 0:
+            return None, None, 0
+        ws = torch.empty(n, dtype=torch.uint8, device=q.device)
     return ws, ws.data_ptr(), n
 
 
