@@ -125,7 +125,8 @@ def main() -> int:
     ap.add_argument("--note", default="", help="description line recorded in a counter summary")
     ap.add_argument("--kernel-match", default="decode_attn_",
                     help="kernel-name substring that picks the profiled kernel in --summarize-counters and "
-                         "--summarize-pmc (default: the decode kernels; prefill_attn_kernel for --prefill runs)")
+                         "--summarize-pmc (default: the decode kernels; for --prefill runs "
+                         "prefill_staged_kernel, or prefill_attn_kernel where the block is too short to stage)")
     ap.add_argument("--summarize-probe", metavar="PROBE_JSON",
                     help="no GPU work: format the JSON line of a --stream-probe run (ceiling per grid, issue "
                          "cost, decode-step time and phases) as text")
@@ -713,6 +714,7 @@ def prefill_bench(args, w: dict) -> int:
     per (query head, query, key) pair. Four layers' caches are cycled."""
     import torch
 
+    from kvint4 import _native as nat
     from kvint4 import ops
 
     B, Hq, Hkv, D, G, Sk = w["B"], w["Hq"], w["Hkv"], w["D"], w["G"], w["ctx"]
@@ -757,6 +759,9 @@ def prefill_bench(args, w: dict) -> int:
     err = (layers[0][5].float() - ops.dense_attention_over_quantized(*layers[0][:5], **kw).float()).abs().max().item()
     if args.calib_copy_mib:
         calibration_copy(args.calib_copy_mib, dev, torch.cuda.current_stream(dev))
+    shape = (B, Hq, Hkv, Sq, D, Sk)
+    staged = (nat.lib().kvq_prefill_attn_staged_workspace_bytes(*shape)
+              != nat.lib().kvq_prefill_attn_workspace_bytes(*shape))
     pairs = sum(min(Sk, Sk - Sq + i + 1) for i in range(Sq))  # admissible (query, key) pairs per head
     flops = 4.0 * B * Hq * D * pairs
     tfs = flops / (ms * 1e-3) / 1e12
@@ -769,7 +774,8 @@ def prefill_bench(args, w: dict) -> int:
                    "kv_heads": Hkv, "head_dim": D, "group_size": G, "context": Sk, "query_tokens": Sq,
                    "causal": True},
         "roofline": {"bound": "mfma", "achieved": round(tfs, 1), "peak": MFMA_BF16_PEAK_TFS, "unit": "TFLOP/s",
-                     "frac": round(tfs / MFMA_BF16_PEAK_TFS, 4), "traffic": None, "kernel": "prefill_attn_kernel"},
+                     "frac": round(tfs / MFMA_BF16_PEAK_TFS, 4), "traffic": None,
+                     "kernel": "stage_kv_kernel + prefill_staged_kernel" if staged else "prefill_attn_kernel"},
         "dequant_flash_ms_per_layer": round(ms_dense, 4), "max_abs_vs_dequant_flash": err,
     }), flush=True)
     return 0
