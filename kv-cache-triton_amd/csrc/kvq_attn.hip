@@ -338,7 +338,8 @@ __device__ __forceinline__ bool ragged_item(const AttnArgs& a, int item, int& b,
   const float T = readlane_f(wave_sum_lane63(lenf), 63);
   const float mx = wave_max(lenf);
   const float slots = (float)a.slots, inv_slots = 1.0f / slots, items = (float)a.items;
-  const int w1 = max(((int)mx + 63) & ~63, 256);
+  // (above the longest length also past 2^24 keys, where mx may be one less)
+  const int w1 = max(((int)mx + 64) & ~63, 256);
   constexpr int NC = 12;
   constexpr float K[NC] = {1.0f, 2.0f, 3.0f, 4.0f, 5.0f, 6.0f, 8.0f, 10.0f, 12.0f, 16.0f, 24.0f, 32.0f};
   int Wc[NC];
@@ -1735,10 +1736,6 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
 // workgroup per CU), 44 without the mixed chunk order below.
 constexpr int kBlockRows = 16;
 constexpr int kBlockWaves = 4;
-#ifndef F32MR
-#define F32MR 8
-#endif
-constexpr int kF32BlockMinRows = F32MR;
 
 template <int D, bool PAGED>
 __global__ __launch_bounds__(64 * kBlockWaves) void decode_attn_f32_block_kernel(const AttnArgs a) {

@@ -178,7 +178,8 @@ def quantize_kv_into(
     dtypes or devices, or none on a GPU) take two."""
     cap = min(k_packed.shape[2], k_scales.shape[2]) if k_packed.dim() == 4 and k_scales.dim() == 4 else -1
     if (not k.is_cuda or k.shape != v.shape or k.dtype != v.dtype or k.device != v.device
-            or k_scales.dtype != v_scales.dtype or v_packed.dim() != 4 or v_scales.dim() != 4 or min(v_packed.shape[2], v_scales.shape[2]) != cap):
+            or k_scales.dtype != v_scales.dtype or v_packed.dim() != 4 or v_scales.dim() != 4
+            or min(v_packed.shape[2], v_scales.shape[2]) != cap):
         quantize_into(k, k_packed, k_scales, group_size, write_pos)
         quantize_into(v, v_packed, v_scales, group_size, write_pos)
         return
