@@ -300,6 +300,11 @@ class _Workspaces:
                 self._bufs[key] = buf
             return buf
 
+    def too_small(self, nbytes: int) -> bool:
+        """Whether this thread's ``using_workspace`` buffer holds less than nbytes."""
+        own = getattr(self._local, "buf", None)
+        return own is not None and own.numel() < nbytes
+
     @contextlib.contextmanager
     def using(self, buf: torch.Tensor):
         if buf.dtype != torch.uint8 or buf.dim() != 1:
@@ -377,8 +382,11 @@ def _plan(q: torch.Tensor, B: int, Hq: int, n_kv_heads: int, Sq: int, D: int, s_
     lengths, by which the splits may be dealt to the sequences."""
     if n_split is not None and n_split < 1:
         raise ValueError("n_split must be >= 1")
-    n, ws_bytes = nat.host().plan(B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, _num_cus(q.device), n_split or 0,
-                                   1 if lengths else 0)
+    shape = (B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, _num_cus(q.device), n_split or 0)
+    n, ws_bytes = nat.host().plan(*shape, 1 if lengths else 0)
+    if lengths and _workspaces.too_small(ws_bytes):
+        # a workspace of the caller's that holds equal splits only
+        n, ws_bytes = nat.host().plan(*shape, 0)
     if n < 0:
         nat.check(n, "kvq_decode_attn_num_splits")
     if ws_bytes < 0:

@@ -156,3 +156,22 @@ def test_plan_rule_and_workspace_bound():
         for Hq, Hkv in ((32, 8), (8, 1), (64, 8), (4, 4), (16, 2)):
             n = plan(B, 1 << 17, Hq, Hkv)
             assert n <= lib.kvq_decode_attn_workspace_bytes(B, Hq, Hkv, 1, 128, bf, bf, 64)
+
+
+def test_workspace_of_the_equal_splits_is_still_enough():
+    """A workspace that the caller sized for the library's equal splits: the
+    call takes them, with the bytes of by_length = False."""
+    B, Hq, Hkv, cap, G = 32, 32, 8, 8192, 32
+    g = torch.Generator(device=DEV).manual_seed(32)
+    n = nat.lib().kvq_decode_attn_num_splits(B, Hq, Hkv, 1, 128, cap, nat.KVQ_BF16, nat.KVQ_BF16, ops._num_cus(DEV))
+    size = ops.decode_workspace_bytes(B, Hq, Hkv, 128, torch.bfloat16, torch.bfloat16, n_split=n)
+    assert size < nat.lib().kvq_decode_attn_by_length_workspace_bytes(B, Hq, Hkv, 1, 128, cap, nat.KVQ_BF16, nat.KVQ_BF16)
+    cache = _cache(B, Hkv, cap, G, "bf16", g)
+    pos = _lengths("mixed", B, cap - 10, g).clamp(min=0)
+    q = torch.randn(B, Hq, 1, 128, generator=g, device=DEV).bfloat16()
+    k, v = (torch.randn(B, Hkv, 1, 128, generator=g, device=DEV).bfloat16() for _ in range(2))
+    kw = dict(n_kv_heads=Hkv, group_size=G, sm_scale=0.0884)
+    want = ops.decode_step(q, k, v, *cache, pos, by_length=False, **kw)
+    with ops.using_workspace(torch.zeros(max(size, 16), dtype=torch.uint8, device=DEV)):
+        got = ops.decode_step(q, k, v, *cache, pos, **kw)
+    assert torch.equal(got, want)
