@@ -40,34 +40,10 @@ MAX_FUSED_ROWS = 1024
 # flash SDPA.
 PREFILL_MIN_ROWS = 64
 PREFILL_MIN_WORK = 1 << 20
-# With several units (batch x KV heads) the launch is large at fewer rows x
-# keys: the fused kernel's time grows with units x keys x ceil(rows / 8), the
-# prefill kernel's with units x keys x ceil(rows / 64). From 48 rows the line
-# is units x rows x keys = 2^22, from 32 rows (four passes of the fused kernel
-# against one of a half-filled row block) 2^24. Measured, fused / prefill (us;
-# GQA 4, D = 128 unless stated): 8 units 64 rows 8200 keys 23.8 / 22.3, 256
-# rows 2048 keys 19.8 / 18.4, below the line 1024 keys 13.5 / 15.5; 32 units
-# 64 rows 2048 keys 21.5 / 18.3, below 1024 keys 14.0 / 15.4; 128 units 256
-# rows 1024 keys 173 / 43; 32 rows, 128 units, 4096 keys 66 / 47, below 512
-# keys 19.0 / 18.3 and (8 units) 32K keys 35.0 / 36.9; 200 units of D = 64,
-# 32 rows, 4096 keys 77 / 59.
-PREFILL_MIN_TOTAL = 1 << 22
-PREFILL_MIN_TOTAL_32 = 1 << 24
 
 
-def prefill_units(q: torch.Tensor, scales: torch.Tensor, n_kv_heads: int, group_size: int) -> int:
-    """use_prefill_kernel's units of a call: 1 for what the prefill kernel would
-    refuse (the call then goes straight to the kernel that takes it)."""
-    B, Hq, _, D = q.shape
-    ok = (q.dtype != torch.float32 and scales.dtype != torch.float32 and D in (64, 128)
-          and group_size in (32, 64, 128) and D % group_size == 0 and 64 % (Hq // n_kv_heads) == 0)
-    return B * n_kv_heads if ok else 1
-
-
-def use_prefill_kernel(rows: int, Sk: int, units: int = 1) -> bool:
-    if rows >= PREFILL_MIN_ROWS and rows * Sk >= PREFILL_MIN_WORK:
-        return True
-    return rows >= 32 and units * rows * Sk >= (PREFILL_MIN_TOTAL if rows >= 48 else PREFILL_MIN_TOTAL_32)
+def use_prefill_kernel(rows: int, Sk: int) -> bool:
+    return rows >= PREFILL_MIN_ROWS and rows * Sk >= PREFILL_MIN_WORK
 
 
 def dense_fast_path(q: torch.Tensor, seq_lens: torch.Tensor | None) -> bool:
@@ -689,7 +665,7 @@ def attention_over_quantized(
     B, Hq, Sq, D = q.shape
     Sk = k_packed.shape[2]
     rows = (Hq // n_kv_heads) * Sq
-    if seq_lens is None and use_prefill_kernel(rows, Sk, prefill_units(q, k_scales, n_kv_heads, group_size)):
+    if seq_lens is None and use_prefill_kernel(rows, Sk):
         try:
             return prefill_attention(q, k_packed, k_scales, v_packed, v_scales, n_kv_heads=n_kv_heads,
                                      group_size=group_size, is_causal=is_causal, sm_scale=sm_scale)

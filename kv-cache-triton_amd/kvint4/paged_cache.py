@@ -365,10 +365,7 @@ class PagedQuantizedKVCache:
         S = max(lens, default=0)
         uniform = all(n == S for n in lens)
         dense_fast = ops.dense_fast_path(query_states, None if uniform else seq_lens)
-        # a captured block of few rows stays on the kernel that reads its lengths on the device at each replay
-        capturing = query_states.is_cuda and torch.cuda.is_current_stream_capturing()
-        units = 1 if capturing else ops.prefill_units(query_states, pools[1], n_kv_heads, self.group_size)
-        if self.page_size >= 64 and uniform and ops.use_prefill_kernel(rows, S, units):
+        if self.page_size >= 64 and uniform and ops.use_prefill_kernel(rows, S):
             try:
                 return ops.prefill_attention_paged(
                     query_states, *pools, pt, S, n_kv_heads=n_kv_heads, group_size=self.group_size,

@@ -1,6 +1,10 @@
-"""Query blocks of a batch on both sides of the lines at which units x rows x keys sends them to the prefill kernel
-instead of the fused decode kernel: either route meets the float64 oracle's bar (2e-2), on the contiguous and the paged
-cache, and the rule never takes a block away from the prefill kernel that a single unit's rows and keys already give it."""
+"""Query blocks that the fused decode kernel takes (fewer than 64 rows per KV head, or rows x keys below the prefill
+kernel's line) keep its precision whatever the batch: K and V codes stay exact there and their scales are fp32, where
+the prefill kernel rounds dequantized K and V to 16 bits.
+
+Bars, relative to the outputs' norm against float64 attention over the cache: 3e-3 for bf16 and 4e-4 for fp16. What the
+fused kernel narrows is the weight p * v_scale and the output (2^-9 each in bf16, 2^-12 and 2^-12 in fp16: measured
+2.0e-3 and 2.3e-4); the prefill kernel's roundings of K and V measure 6e-3 and 8.5e-4 on keys with outlier channels."""
 
 from __future__ import annotations
 
@@ -10,14 +14,16 @@ import torch
 from kvint4 import ops
 from kvint4.paged_cache import PagedQuantizedKVCache
 
+BARS = {torch.bfloat16: 3e-3, torch.float16: 4e-4}
 
-def test_rule_only_adds():
-    for rows in (1, 31, 32, 47, 48, 63, 64, 100, 1024, 70000):
-        for Sk in (0, 64, 1000, 4096, 16384, 65536):
-            for units in (1, 8, 128):
-                got = ops.use_prefill_kernel(rows, Sk, units)
-                assert got or not ops.use_prefill_kernel(rows, Sk)
-                assert not got or rows >= 32
+
+def test_more_kv_heads_than_query_heads_is_refused():
+    """The library's own refusal, as for any other shape it does not take (without a GPU: that there is none)."""
+    q = torch.zeros(1, 4, 8, 64, dtype=torch.float16)
+    p = torch.zeros(1, 8, 16, 32, dtype=torch.uint8)
+    s = torch.zeros(1, 8, 16, 2, dtype=torch.float16)
+    with pytest.raises((ValueError, RuntimeError)):
+        ops.attention_over_quantized(q, p, s, p, s, n_kv_heads=8, group_size=32, is_causal=True, sm_scale=0.1)
 
 
 def _want(q, cache, G, n_kv):
@@ -42,34 +48,33 @@ def _want(q, cache, G, n_kv):
 
 
 CASES = [
-    # B, Hq, Hkv, Sq, Sk, D, dtype, prefill route
-    (4, 8, 2, 16, 8192, 128, torch.bfloat16, True),    # 64 rows: 2^22 exactly
-    (4, 8, 2, 16, 8191, 128, torch.bfloat16, False),   # one key short of it
-    (8, 12, 12, 47, 1100, 64, torch.float16, False),   # 47 rows: the line is 2^24
-    (8, 12, 12, 48, 1100, 64, torch.float16, True),    # 48 rows: past 2^22
-    (4, 8, 8, 32, 16384, 64, torch.bfloat16, True),    # 32 rows: 2^24 exactly
-    (4, 8, 8, 31, 17000, 64, torch.bfloat16, False),   # 31 rows: past 2^24, never
+    # B, Hq, Hkv, Sq, Sk, D, dtype
+    (1, 32, 8, 8, 8200, 128, torch.bfloat16),    # 32 rows, one sequence
+    (16, 32, 8, 8, 4096, 128, torch.bfloat16),   # 32 rows, a batch
+    (16, 32, 8, 12, 2100, 128, torch.float16),   # 48 rows
+    (16, 32, 8, 16, 1000, 128, torch.bfloat16),  # 64 rows below the prefill kernel's rows x keys
+    (8, 12, 12, 48, 1100, 64, torch.float16),    # MHA, D = 64
+    (8, 12, 12, 63, 1100, 64, torch.bfloat16),
 ]
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("paged", [False, True])
-@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,dtype,prefill", CASES)
-def test_blocks_at_the_lines(monkeypatch, B, Hq, Hkv, Sq, Sk, D, dtype, prefill, paged):
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,dtype", CASES)
+def test_blocks_keep_the_fused_kernels_precision(B, Hq, Hkv, Sq, Sk, D, dtype, paged):
     dev, G = torch.device("cuda:0"), 32
     g = torch.Generator(device=dev).manual_seed(Sk + Sq)
-    q, k, v = (torch.randn(B, h, s, D, generator=g, device=dev).to(dtype) for h, s in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk)))
+    q, k, v = (torch.randn(B, h, s, D, generator=g, device=dev) for h, s in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk)))
+    k[..., [(5 + 13 * i) % D for i in range(8)]] *= 8.0  # outlier channels, as trained models' keys have them
+    q, k, v = q.to(dtype), k.to(dtype), v.to(dtype)
     dense = (*ops.quantize(k, G, dtype), *ops.quantize(v, G, dtype))
-    taken = []
-    for name in ("prefill_attention", "prefill_attention_paged"):
-        real = getattr(ops, name)
-        monkeypatch.setattr(ops, name, lambda *a, _f=real, **kw: (taken.append(1), _f(*a, **kw))[1])
-    kw = dict(n_kv_heads=Hkv, group_size=G, is_causal=True, sm_scale=D ** -0.5)
     if paged:
         cache = PagedQuantizedKVCache(group_size=G, page_size=128)
         cache.append(k, v, 0)
         out = cache.attend(q, 0, n_kv_heads=Hkv, is_causal=True, scale=D ** -0.5)
     else:
-        out = ops.attention_over_quantized(q, *dense, **kw)
-    assert bool(taken) == prefill
-    assert (out.double() - _want(q, dense, G, Hkv)).abs().max().item() <= 2e-2
+        out = ops.attention_over_quantized(q, *dense, n_kv_heads=Hkv, group_size=G, is_causal=True, sm_scale=D ** -0.5)
+    want = _want(q, dense, G, Hkv)
+    err = ((out.double() - want).norm() / want.norm()).item()
+    print(f"rows {Hq // Hkv * Sq} keys {Sk} batch {B} {dtype}: relative error {err:.2e}", flush=True)
+    assert err <= BARS[dtype]
