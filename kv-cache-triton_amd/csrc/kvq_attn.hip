@@ -1920,14 +1920,16 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decode_attn_f32_block_kernel
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
     }
-    // scores in base 2; excluded keys -inf (weight exactly 0)
+    // scores in base 2; excluded keys -inf (weight exactly 0), and keys whose
+    // score is not a number (a NaN scale) too, as in the VALU kernel
     const int klim = have ? lim - 64 * tile - 4 * g : 0;
     float mx = -__builtin_inff();
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        st[kb][r] = 16 * kb + r < klim ? st[kb][r] * a.scale_log2 : -__builtin_inff();
+        const float s = st[kb][r] * a.scale_log2;
+        st[kb][r] = 16 * kb + r < klim && s > kNeg ? s : -__builtin_inff();
         mx = fmaxf(mx, st[kb][r]);
       }
     mx = fmaxf(mx, __shfl_xor(mx, 16));

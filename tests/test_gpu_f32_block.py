@@ -137,3 +137,25 @@ def test_f32_block_paged_with_missing_page():
         want = _want(q[b:b + 1], _dequant64(kp[:, rows], ks[:, rows], G, D)[None],
                      _dequant64(vp[:, rows], vs[:, rows], G, D)[None], D ** -0.5, False)
         _check(out[b:b + 1], want)
+
+
+def test_f32_block_nan_key_scale():
+    """A key whose score is not a number weighs nothing and the row keeps its other keys, as on the VALU kernel."""
+    B, H, Sq, Sk, D, G, bad = 1, 12, 100, 300, 64, 32, 130
+    g = torch.Generator(device=DEV).manual_seed(12)
+    q = torch.randn(B, H, Sq, D, generator=g, device=DEV)
+    kp, ks, vp, vs = _kv(B, H, Sk, D, G, "f16", g)
+    ks[:, :, bad, 1] = float("nan")
+    kw = dict(n_kv_heads=H, group_size=G, is_causal=True, sm_scale=D ** -0.5)
+    out = ops.fused_decode_attention(q, kp, ks, vp, vs, **kw)
+    keep = [t for t in range(Sk) if t != bad]  # (a causal row before the key, too, has the same keys without it)
+    want = torch.empty(B, H, Sq, D, dtype=torch.float64, device=DEV)
+    k, v = _dequant64(kp, ks, G, D), _dequant64(vp, vs, G, D)
+    for h in range(H):
+        s = q[0, h].double() @ k[0, h][keep].T.contiguous() * D ** -0.5
+        lim = Sk - Sq + torch.arange(Sq, device=DEV)[:, None]
+        s = s.masked_fill(torch.tensor(keep, device=DEV)[None] > lim, float("-inf"))
+        want[0, h] = torch.softmax(s, -1) @ v[0, h][keep]
+    _check(out, want)
+    valu = ops.fused_decode_attention(q, kp, ks, vp, vs, n_split=2, **kw)
+    assert (out - valu).abs().max().item() <= 2e-5
