@@ -1808,21 +1808,12 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decode_attn_f32_block_kernel
 
   // raw codes and scales of a tile: K of keys 16 kb + n, V of keys 16 kb +
   // 4 g + r. Keys past the sequence read its last row (inside the tile, hence
-  // in its page) and are masked; a paged tile without a block reads pool row 0
-  // and is masked.
+  // in its page) and are masked. dl: the tile's pool rows less its keys.
   uint32_t kw[4][KW], vw[4][4];
   float ksc[4], vsc[4][4];
-  bool have = false;  // a block holds the tile in kw / vw
-  auto load_tile = [&](int tile) {
+  auto load_tile = [&](int tile, uint32_t dl) {
     const int t0 = 64 * tile;
-    uint32_t dl = 0u;
-    bool ok = true;
-    if constexpr (PAGED) page_delta(a, bt_b, (uint32_t)t0, dl, ok);
-    have = ok;
-    auto row = [&](int t) -> uint32_t {
-      const uint32_t tc = (uint32_t)min(t, last_tok);
-      return ok ? tc + dl : 0u;
-    };
+    auto row = [&](int t) -> uint32_t { return (uint32_t)min(t, last_tok) + dl; };
     uint32_t kr[4], vr[4][4];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
@@ -1895,7 +1886,16 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decode_attn_f32_block_kernel
   for (int db = 0; db < VD; ++db) o[db] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = kNeg, l_run = 0.0f;
   for (int tile = wave; tile < ntiles; tile += NW) {
-    load_tile(tile);
+    uint32_t dl = 0u;
+    if constexpr (PAGED) {
+      // a tile whose page has no block is passed over: no keys (and what a
+      // pool's unused rows hold, NaN scales perhaps, does not reach the
+      // products, where a weight of 0 would not stop it)
+      bool ok;
+      page_delta(a, bt_b, (uint32_t)(64 * tile), dl, ok);
+      if (!__builtin_amdgcn_readfirstlane((int)ok)) continue;
+    }
+    load_tile(tile, dl);
     f32x4_t st[4];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) st[kb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1922,7 +1922,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decode_attn_f32_block_kernel
     }
     // scores in base 2; excluded keys -inf (weight exactly 0), and keys whose
     // score is not a number (a NaN scale) too, as in the VALU kernel
-    const int klim = have ? lim - 64 * tile - 4 * g : 0;
+    const int klim = lim - 64 * tile - 4 * g;
     float mx = -__builtin_inff();
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)

@@ -159,3 +159,30 @@ def test_f32_block_nan_key_scale():
     _check(out, want)
     valu = ops.fused_decode_attention(q, kp, ks, vp, vs, n_split=2, **kw)
     assert (out - valu).abs().max().item() <= 2e-5
+
+
+def test_f32_block_missing_page_reads_no_pool_row():
+    """A tile without a block contributes nothing whatever the pool's unused rows (row 0 among them) hold."""
+    B, H, Sq, D, G, P, S = 2, 12, 60, 64, 32, 64, 400
+    g = torch.Generator(device=DEV).manual_seed(14)
+    q = torch.randn(B, H, Sq, D, generator=g, device=DEV)
+    cols = -(-S // P)
+    nb = B * cols + 2
+    kp, ks, vp, vs = (t[0] for t in _kv(1, H, nb * P, D, G, "f16", g))
+    table = 1 + torch.randperm(nb - 1, generator=torch.Generator().manual_seed(2))[: B * cols].view(B, cols)
+    table = table.to(DEV, torch.int32)
+    table[0, 0], table[1, 2], table[1, 6] = -1, -1, -1
+    used = torch.zeros(nb, dtype=torch.bool, device=DEV)
+    used[table[table >= 0].long()] = True
+    for s in (ks, vs):
+        s[:, ~used.repeat_interleave(P)] = float("nan")
+    pt = ops.PageTable(table, P, nb)
+    out = ops.fused_decode_attention_paged(q, kp, ks, vp, vs, pt, n_kv_heads=H, group_size=G, is_causal=False,
+                                           sm_scale=D ** -0.5, seq_len=S)
+    t = torch.arange(S, device=DEV)
+    for b in range(B):
+        rows = table[b, t // P].long() * P + t % P
+        rows = rows[table[b, t // P] >= 0]
+        want = _want(q[b:b + 1], _dequant64(kp[:, rows], ks[:, rows], G, D)[None],
+                     _dequant64(vp[:, rows], vs[:, rows], G, D)[None], D ** -0.5, False)
+        _check(out[b:b + 1], want)
