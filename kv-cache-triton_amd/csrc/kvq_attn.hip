@@ -1743,7 +1743,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decode_attn_f32_block_kernel
   constexpr int KD = D / 4;   // K dims per lane
   constexpr int VD = D / 16;  // V dims per lane
   constexpr int KW = KD / 8;  // K code dwords per lane
-  __shared__ float o_lds[NW][ROWS][D];
+  __shared__ __attribute__((aligned(16))) float o_lds[NW][ROWS][D];  // (read as float4 by the fold)
   __shared__ __attribute__((aligned(16))) float ml_lds[NW][ROWS][2];
 
   const int tid = threadIdx.x, lane = tid & 63;
