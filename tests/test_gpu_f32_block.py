@@ -186,3 +186,37 @@ def test_f32_block_missing_page_reads_no_pool_row():
         want = _want(q[b:b + 1], _dequant64(kp[:, rows], ks[:, rows], G, D)[None],
                      _dequant64(vp[:, rows], vs[:, rows], G, D)[None], D ** -0.5, False)
         _check(out[b:b + 1], want)
+
+
+@pytest.mark.parametrize("H,Sq,Sk,causal", [
+    (12, 1000, 1000, True),    # 756 units: both chunk orders, the change of order inside a head's chunks
+    (3, 4105, 300, False),     # a head's last chunk is unit 256: the second head starts just past it
+    (3, 4105, 4200, True),
+])
+def test_f32_block_many_units(H, Sq, Sk, causal):
+    """Launches past 256 units, where every other 256 units' heads take their chunks in the other order: each chunk is
+    written once, whichever order it is taken in (the output starts as NaN)."""
+    D, G = 64, 32
+    g = torch.Generator(device=DEV).manual_seed(Sq + Sk)
+    q = torch.randn(1, H, Sq, D, generator=g, device=DEV)
+    kp, ks, vp, vs = _kv(1, H, Sk, D, G, "f16", g)
+    want = _want(q, _dequant64(kp, ks, G, D), _dequant64(vp, vs, G, D), D ** -0.5, causal)
+    out = torch.full_like(q, float("nan"))
+    ops.fused_decode_attention(q, kp, ks, vp, vs, n_kv_heads=H, group_size=G, is_causal=causal, sm_scale=D ** -0.5,
+                               out=out)
+    _check(out, want)
+
+
+@pytest.mark.parametrize("sd", ["bf16", "f32"])
+def test_f32_block_largest_key_scales(sd):
+    """Keys near the largest fp32 value (scales above 2^124) under small queries: a dequantized key times 16 would
+    overflow, its scores do not."""
+    B, H, Sq, Sk, D, G = 1, 12, 100, 300, 64, 32
+    g = torch.Generator(device=DEV).manual_seed(15)
+    q = torch.randn(B, H, Sq, D, generator=g, device=DEV) * 1e-38
+    kp, ks = ops.quantize(torch.randn(B, H, Sk, D, generator=g, device=DEV).clamp(-3, 3) * 1.13e38, G, SDT[sd])
+    vp, vs = ops.quantize(torch.randn(B, H, Sk, D, generator=g, device=DEV), G, SDT[sd])
+    assert ks.float().max().item() > 2.0 ** 125
+    want = _want(q, _dequant64(kp, ks, G, D), _dequant64(vp, vs, G, D), D ** -0.5, True)
+    _check(ops.fused_decode_attention(q, kp, ks, vp, vs, n_kv_heads=H, group_size=G, is_causal=True,
+                                      sm_scale=D ** -0.5), want)
