@@ -779,6 +779,12 @@ void prefill_staged_kernel(const PrefillArgs a) {
   const int tps = (tiles_all + a.n_split - 1) / a.n_split;
   const int tile_lo = sp * tps;
   const int n = min(tiles_all, tile_lo + tps) - tile_lo;  // tiles of this workgroup (<= 0: none)
+  // the wave's own: past its last row's last key it only moves images. (Their
+  // weights would all be 0, but 0 times an infinite or NaN value is NaN: a key
+  // may reach no row block but those of the waves that attend its tile.)
+  const int r_wave = min(R0 + 32, a.Sq * a.ratio) - 1;
+  const int kend_wave = r_wave < R0 ? 0 : clamp_keys(a.causal ? a.Sk - a.Sq + r_wave / a.ratio + 1 : a.Sk);
+  const int n_wave = max(min(n, (kend_wave + kKeys - 1) / kKeys - tile_lo), 0);
 
   // queries as the B operand: lane (ln, lg) holds dims 16 kk + 8 lg .. + 7 of
   // its row (rows past Sq are zero); the sign of sm_scale goes into them and
@@ -922,15 +928,21 @@ void prefill_staged_kernel(const PrefillArgs a) {
     scores(k_lds[0], sA);
     __syncthreads();  // every wave has read K buffer 0, which tile 0 refills
     int i = 0;
-    for (; i + 1 < n; i += 2) {
+    for (; i + 1 < n_wave; i += 2) {
       step(sA, sB, pB, pA, i, 0);
       step(sB, sA, pA, pB, i + 1, 1);
     }
-    if (i < n) {
+    if (i < n_wave) {
       step(sA, sB, pB, pA, i, 0);
       values(v_lds[0], pA);
+      ++i;
     } else {
       values(v_lds[1], pB);
+    }
+    for (; i < n; ++i) {  // tiles that only other waves attend
+      fetch(0, i + 2, k_lds[i & 1]);
+      fetch(1, i, v_lds[i & 1]);
+      arrive();
     }
   }
 

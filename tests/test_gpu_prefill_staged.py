@@ -179,3 +179,52 @@ def test_staged_units_in_groups():
     b = _call(q, kp, ks, vp, vs, Hkv, G, True, D ** -0.5, False)
     # outputs average thousands of values (|out| < 0.2): two bf16 roundings of them and of the weights
     assert (a.float() - b.float()).abs().max().item() <= 2e-3
+
+
+def _attended(q, Sk, ratio, bad, causal):
+    """[Sq]: whether a query position attends key `bad`."""
+    i = torch.arange(q.shape[2], device=DEV)
+    return (Sk - q.shape[2] + i >= bad) if causal else torch.ones_like(i, dtype=torch.bool)
+
+
+@pytest.mark.parametrize("what,value", [("key", float("nan")), ("key", float("inf")), ("value", float("nan")),
+                                        ("value", float("inf")), ("value", float("-inf"))])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,dtype,bad", [
+    (1, 32, 8, 2048, 2048, 128, "bf16", 1000),   # eight waves per workgroup
+    (1, 32, 8, 530, 1088, 128, "f16", 700),      # four; the key's tile begins in the second half of their rows
+    (4, 16, 16, 1030, 1030, 64, "bf16", 700),    # MHA, D 64, eight waves; the same
+    (1, 4, 1, 777, 9001, 128, "f16", 8500),      # a split over keys
+])
+def test_staged_non_finite_scales(what, value, B, Hq, Hkv, Sq, Sk, D, dtype, bad):
+    """One key with a scale that is not finite: its rows' outputs are not finite, as on the unstaged kernel, and every
+    row that the unstaged kernel keeps finite (a wave's masked keys share matrix products with the rows before them, in
+    both kernels) stays finite and right."""
+    G, ratio = 32, Hq // Hkv
+    g = torch.Generator(device=DEV).manual_seed(Sk + bad)
+    q = torch.randn(B, Hq, Sq, D, generator=g, device=DEV).to(TDT[dtype])
+    kp, ks, vp, vs = _quantized(B, Hkv, Sk, D, dtype, G, g)
+    want = _want(q, _dequant64(kp, ks, G, D), _dequant64(vp, vs, G, D), D ** -0.5, True)
+    (ks if what == "key" else vs)[:, :, bad] = value
+    a = _call(q, kp, ks, vp, vs, Hkv, G, True, D ** -0.5, True)
+    b = _call(q, kp, ks, vp, vs, Hkv, G, True, D ** -0.5, False)
+    fa, fb = torch.isfinite(a).all(-1), torch.isfinite(b).all(-1)
+    attends = _attended(q, Sk, ratio, bad, True)
+    print(f"rows that attend the key {attends.sum().item()}, not finite: staged {(~fa[0, 0]).sum().item()}, "
+          f"unstaged {(~fb[0, 0]).sum().item()}", flush=True)
+    assert not fa[:, :, attends].any() and not fb[:, :, attends].any()
+    assert fa[fb].all()
+    assert fa[:, :, ~attends].any()
+    assert (a.double() - want).abs()[fa].max().item() <= 2e-2
+
+
+def test_staged_largest_scales():
+    """Key scales above 2^125 (-8 times them overflows) under small queries and a small softmax scale."""
+    B, Hq, Hkv, Sq, Sk, D, G = 1, 32, 8, 520, 1088, 128, 32
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q = (torch.randn(B, Hq, Sq, D, generator=g, device=DEV) * 1e-10).bfloat16()
+    kp, ks, vp, vs = _quantized(B, Hkv, Sk, D, "bf16", G, g)
+    kp, ks = ops.quantize((torch.randn(B, Hkv, Sk, D, generator=g, device=DEV).clamp(-3, 3) * 1.1e38).bfloat16(), G,
+                          torch.bfloat16)
+    assert ks.float().max().item() > 2.0 ** 125
+    want = _want(q, _dequant64(kp, ks, G, D), _dequant64(vp, vs, G, D), 8e-30, True)
+    _compare(q, kp, ks, vp, vs, Hkv, G, True, 8e-30, want)
