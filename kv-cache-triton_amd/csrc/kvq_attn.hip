@@ -1920,16 +1920,14 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decode_attn_f32_block_kernel
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
     }
-    // scores in base 2; excluded keys -inf (weight exactly 0), and keys whose
-    // score is not a number (a NaN scale) too, as in the VALU kernel
+    // scores in base 2; excluded keys -inf (weight exactly 0)
     const int klim = lim - 64 * tile - 4 * g;
     float mx = -__builtin_inff();
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float s = st[kb][r] * a.scale_log2;
-        st[kb][r] = 16 * kb + r < klim && s > kNeg ? s : -__builtin_inff();
+        st[kb][r] = 16 * kb + r < klim ? st[kb][r] * a.scale_log2 : -__builtin_inff();
         mx = fmaxf(mx, st[kb][r]);
       }
     mx = fmaxf(mx, __shfl_xor(mx, 16));
@@ -1946,7 +1944,12 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decode_attn_f32_block_kernel
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float p = __builtin_amdgcn_exp2f(st[kb][r] - m_run);
+        // clamped to [0, 1], where it lies in any case, because that gives a
+        // key whose score is not a number (a NaN scale; the max passes over
+        // it) the weight 0, as in the VALU kernel: an output modifier of the
+        // exponential, no instruction (a compare and select per score took
+        // 3.5 % at D = 64)
+        const float p = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(st[kb][r] - m_run), 0.0f, 1.0f);
         l_run += p;
         uint32_t lo, hi;
         halves(vw[kb][r], lo, hi);
