@@ -21,6 +21,7 @@ HOST_PATH = os.path.join(_HERE, "_kvq_host.so")
 
 KVQ_BF16, KVQ_F16, KVQ_F32 = 0, 1, 2
 KVQ_OK, KVQ_EINVAL, KVQ_ESPACE, KVQ_EHIP, KVQ_EUNSUP = 0, -1, -2, -3, -4
+KVQ_SPLIT_BY_LENGTH = 1 << 30
 
 # The argument lists below are those of major version 2 (KVQ_VERSION in
 # include/kvint4.h: major*10000 + minor*100 + patch); a library of another

@@ -35,7 +35,9 @@ class _LayerQuantizedKV:
     """Per-layer state. Field names follow the reference
     (models/llama3/kv_cache.py:21-27); the tensors may hold more rows than
     ``seq_len`` (capacity). ``seq_lens`` (device lengths) is set for ragged
-    layers and after ``make_static``."""
+    layers and after ``make_static``. ``lag`` is what a ragged layer's host
+    knows of them, where it knows it: by how many rows the sequences fall short
+    of ``seq_len``, (all together, the longest)."""
 
     k_packed: torch.Tensor
     k_scales: torch.Tensor
@@ -43,11 +45,17 @@ class _LayerQuantizedKV:
     v_scales: torch.Tensor
     seq_len: int
     seq_lens: Optional[torch.Tensor] = None
-    ragged: bool = False  # the sequences' lengths differ (load_ragged)
+    lag: Optional[tuple[int, int]] = None
 
     @property
     def capacity(self) -> int:
         return int(self.k_packed.shape[2])
+
+
+def _lag(lengths: torch.Tensor, seq_len: int) -> tuple[int, int]:
+    """_LayerQuantizedKV.lag of sequences of these lengths (a host tensor)."""
+    lens = [min(max(int(n), 0), seq_len) for n in lengths.flatten().tolist()]
+    return seq_len * len(lens) - sum(lens), seq_len - max(lens, default=seq_len)
 
 
 def _round_up(n: int, m: int) -> int:
@@ -240,11 +248,17 @@ class QuantizedKVCacheBase:
         start = prev.seq_len
         layer = self._ensure_layer(key_states, layer_idx, start + 1)
         pos = layer.seq_lens if layer.seq_lens is not None else start
+        by_length = False
+        if layer.lag is not None:
+            B, Hq, _, D = query_states.shape
+            by_length = ops.by_length_pays(B, Hq, n_kv_heads, D, query_states.dtype, layer.k_scales.dtype,
+                                           layer.capacity, B * start - layer.lag[0], start - layer.lag[1],
+                                           ops._num_cus(query_states.device))
         try:
             out = ops.decode_step(
                 query_states, key_states, value_states,
                 layer.k_packed, layer.k_scales, layer.v_packed, layer.v_scales, pos,
-                n_kv_heads=n_kv_heads, group_size=self.group_size, sm_scale=scale, by_length=layer.ragged,
+                n_kv_heads=n_kv_heads, group_size=self.group_size, sm_scale=scale, by_length=by_length,
             )
         except _native.KVQUnsupported:
             return None
@@ -271,7 +285,8 @@ class QuantizedKVCacheBase:
         self._append_quantized(key_states, value_states, layer_idx)
         layer = self._layers[layer_idx]
         layer.seq_lens = lengths.to(device=key_states.device, dtype=torch.int32).clone()
-        layer.ragged = True
+        if not lengths.is_cuda:  # (lengths on the device are not waited for)
+            layer.lag = _lag(lengths, layer.seq_len)
 
     def get_seq_lens(self, layer_idx: int) -> Optional[torch.Tensor]:
         """Per-sequence lengths of a ragged layer (device int32 [B]) or None."""
@@ -309,6 +324,7 @@ class QuantizedKVCacheBase:
             layer.k_packed, layer.k_scales, layer.v_packed, layer.v_scales = bufs
             if layer.seq_lens is not None:
                 layer.seq_lens = layer.seq_lens[idx].contiguous()
+            layer.lag = None
 
     def _batch_size(self) -> int:
         return int(next(iter(self._layers.values())).k_packed.shape[0]) if self._layers else 0
@@ -353,6 +369,7 @@ class QuantizedKVCacheBase:
                     layer.seq_lens.add_(max_length).clamp_(min=0)
                 else:
                     layer.seq_lens.clamp_(max=keep)
+                    layer.lag = None
             layer.seq_len = keep
 
     def nbytes(self) -> int:

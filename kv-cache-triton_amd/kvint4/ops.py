@@ -352,6 +352,37 @@ def _num_cus(device: torch.device) -> int:
     return n
 
 
+# Splits by length cost a launch what its workgroups need to work them out of the
+# lengths, 1.2 to 2 us (up to 5 where the splits take more than one round of
+# workgroups), which lengths that are alike never win back: 2 to 64 sequences of
+# one length, D = 128, GQA 4 and 8, ran 4 to 34 % slower so (32 x 512 tokens of
+# 8K rows 7.5 / 11.3 us). So they are the caller's choice, and the caches, which
+# know their lengths on the host, take them where an equal split of the longest
+# sequence holds twice the keys of a balanced one and 2048 more: of 680 batches
+# measured (lengths spread over up to a factor of 64, one long among short, half
+# and half; capacities 4K to 32K and a quarter of them filled) all 48 inside that
+# line were faster (1.03x to 2.9x, 20 us on average); with 1024 more, 6 of 78
+# were slower, down to 0.87x.
+BY_LENGTH_MIN_KEYS = 2048
+
+
+def by_length_pays(B: int, Hq: int, n_kv_heads: int, D: int, q_dtype: torch.dtype, scale_dtype: torch.dtype,
+                   capacity: int, total: int, longest: int, num_cus: int) -> bool:
+    """Whether splits by length pay for one decode token of B sequences, of
+    `total` cached keys together and `longest` in the longest."""
+    if B < 2 or total == B * longest or Hq < n_kv_heads or n_kv_heads < 1:
+        return False
+    slots = -(-num_cus // (n_kv_heads * -(-(Hq // n_kv_heads) // 8)))  # workgroups per (KV head, 8 query rows)
+    floor = 2 * total / slots + BY_LENGTH_MIN_KEYS
+    if longest < floor:
+        return False
+    shape = (B, Hq, n_kv_heads, 1, D, capacity, nat.DTYPE_CODE[q_dtype], nat.DTYPE_CODE[scale_dtype], num_cus, 0)
+    if nat.host().plan(*shape, 1)[0] != nat.KVQ_SPLIT_BY_LENGTH:
+        return False
+    n = nat.host().plan(*shape, 0)[0]
+    return n > 0 and longest / n >= floor
+
+
 def _plan(q: torch.Tensor, B: int, Hq: int, n_kv_heads: int, Sq: int, D: int, s_max: int,
           qd: int, sd: int, n_split: int | None, lengths: bool) -> tuple[int, int]:
     """(splits, workspace bytes) of a decode launch; `lengths`: it has device
@@ -392,6 +423,7 @@ def fused_decode_attention(
     seq_lens: torch.Tensor | None = None,
     out: torch.Tensor | None = None,
     n_split: int | None = None,
+    by_length: bool = False,
 ) -> torch.Tensor:
     """Launch the fused split-K decode kernel; raises KVQUnsupported for shapes
     it does not handle. q [B, Hq, Sq, D]; K/V codes [B, Hkv, Sk, W] (strided views
@@ -417,7 +449,7 @@ def fused_decode_attention(
         sl_ptr = seq_lens.data_ptr()
     qd = nat.DTYPE_CODE[q.dtype]
     sd = nat.DTYPE_CODE[k_scales.dtype]
-    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, Sk, qd, sd, n_split, sl_ptr is not None)
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, Sk, qd, sd, n_split, by_length and sl_ptr is not None)
     with nat.device_of(q) as stream:
         ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
         rc = nat.host().decode_attn(
@@ -484,7 +516,7 @@ def decode_step(
     sm_scale: float,
     out: torch.Tensor | None = None,
     n_split: int | None = None,
-    by_length: bool = True,
+    by_length: bool = False,
 ) -> torch.Tensor:
     """One decode token in one launch: quantize k_new / v_new [B, Hkv, 1, D]
     into row `position` of the capacity buffers (an int for every sequence, or
@@ -493,9 +525,9 @@ def decode_step(
     [B, Hkv, capacity, .] tensors, written in place; the caller advances its
     lengths. Raises KVQUnsupported for dtype/group combinations the fused
     step does not handle (the caller then quantizes and attends separately).
-    With device positions a batch's splits are dealt to the sequences by their
-    lengths where that pays; `by_length` = False says that the lengths are
-    alike, so that every sequence gets the same splits without working that out."""
+    `by_length` = True, for device positions that differ a lot
+    (by_length_pays): the splits are dealt to the sequences by their lengths
+    instead of the same number to each."""
     B, Hq, Sq, D = q.shape
     if Sq != 1:
         raise nat.KVQUnsupported("decode_step handles one query position")
@@ -843,6 +875,7 @@ def fused_decode_attention_paged(
     seq_len: int | None = None,
     out: torch.Tensor | None = None,
     n_split: int | None = None,
+    by_length: bool = False,
 ) -> torch.Tensor:
     """fused_decode_attention over a paged cache. Sequence b attends its first
     seq_lens[b] tokens (device int32 [B]) or `seq_len` tokens. bf16/fp16
@@ -871,7 +904,7 @@ def fused_decode_attention_paged(
         seq_len = int(seq_len)
         s_max = seq_len
     qd, sd = nat.DTYPE_CODE[q.dtype], nat.DTYPE_CODE[k_scales.dtype]
-    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, n_split, sl_ptr is not None)
+    n_split, ws_bytes = _plan(q, B, Hq, n_kv_heads, Sq, D, s_max, qd, sd, n_split, by_length and sl_ptr is not None)
     with nat.device_of(q) as stream:
         ws_ptr, ws_len = _decode_ws(q, stream, ws_bytes)
         rc = nat.host().decode_attn_paged(
@@ -941,7 +974,7 @@ def decode_step_paged(
     sm_scale: float,
     out: torch.Tensor | None = None,
     n_split: int | None = None,
-    by_length: bool = True,
+    by_length: bool = False,
 ) -> torch.Tensor:
     """decode_step over a paged cache: the new token of sequence b goes to its
     position (int, or device int32 [B] of old lengths) through the block table;

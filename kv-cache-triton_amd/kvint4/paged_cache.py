@@ -282,10 +282,13 @@ class PagedQuantizedKVCache:
         pools = self._pools[layer_idx]
         pt = self._page_table()
         pos = self._seq_lens[layer_idx]
+        B, Hq, _, D = query_states.shape
+        by_length = ops.by_length_pays(B, Hq, n_kv_heads, D, query_states.dtype, pools[1].dtype, pt.capacity, sum(lens),
+                                       max(lens, default=0), ops._num_cus(query_states.device))
         try:
             out = ops.decode_step_paged(query_states, key_states, value_states, *pools, pt, pos,
                                         n_kv_heads=n_kv_heads, group_size=self.group_size, sm_scale=scale,
-                                        by_length=any(n != lens[0] for n in lens))
+                                        by_length=by_length)
         except _native.KVQUnsupported:
             return None
         pos.add_(1)

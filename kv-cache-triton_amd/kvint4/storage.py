@@ -30,7 +30,7 @@ import torch
 from safetensors.torch import load_file, save_file
 
 from . import ops
-from .cache_base import QuantizedKVCacheBase, _LayerQuantizedKV
+from .cache_base import QuantizedKVCacheBase, _lag, _LayerQuantizedKV
 from .paged_cache import PagedQuantizedKVCache
 
 FORMAT = "kvint4-cache"
@@ -118,5 +118,6 @@ def load_cache(path: str, cache: Cache, device: Union[str, torch.device] = "cuda
             continue
         S = parts[0].shape[2]
         ragged = bool((lens != S).any())
-        cache._layers[i] = _LayerQuantizedKV(*parts, S, lens.to(dev) if ragged else None, ragged)
+        cache._layers[i] = _LayerQuantizedKV(*parts, S, lens.to(dev) if ragged else None,
+                                             _lag(lens, S) if ragged else None)
     return cache

@@ -1,7 +1,7 @@
 """GPU parity: decode attention whose splits are dealt to the sequences of a
-batch by their device lengths (KVQ_SPLIT_BY_LENGTH, which the operators plan for batches of 2 to 64
-sequences over large caches) against the same launch with
-equal splits per sequence and against float64 attention.
+batch by their device lengths (KVQ_SPLIT_BY_LENGTH, for batches of 2 to 64
+sequences over large caches, where the caller asks for it) against the same
+launch with equal splits per sequence and against float64 attention.
 
 Both plans run the same tile code and differ in where a sequence is cut and
 in the merge's order: outputs agree within two bf16 / fp16 roundings of the
@@ -23,7 +23,6 @@ import torch
 from kvint4 import _native as nat
 from kvint4 import ops
 
-pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
 BY_LENGTH = 1 << 30  # KVQ_SPLIT_BY_LENGTH
 TDT = {"bf16": torch.bfloat16, "f16": torch.float16}
@@ -70,6 +69,7 @@ CASES = [(2, 32, 8, 4096, "one_long", "bf16", 32), (7, 8, 8, 4100, "mixed", "f16
          (64, 64, 8, 4096, "one_long", "bf16", 128), (12, 64, 8, 5000, "equal", "f16", 32), (20, 16, 4, 5000, "mixed", "bf16", 32)]
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,Hq,Hkv,cap,kind,dtype,G", CASES)
 def test_step_and_attention_by_length(B, Hq, Hkv, cap, kind, dtype, G):
     g = torch.Generator(device=DEV).manual_seed(B * cap)
@@ -101,6 +101,7 @@ def test_step_and_attention_by_length(B, Hq, Hkv, cap, kind, dtype, G):
         assert (sa[i, :, 0].double() - _want(q[i, :, 0], k64[i], v64[i], m, 128 ** -0.5)).abs().max().item() <= 2e-2
 
 
+@pytest.mark.gpu
 def test_paged_step_by_length_and_graph_replays():
     """A paged batch: equal to the equal-splits plan; then captured, and replayed while the lengths change."""
     B, Hq, Hkv, P, cols, G = 6, 32, 8, 64, 64, 32
@@ -141,6 +142,7 @@ def test_paged_step_by_length_and_graph_replays():
             assert torch.equal(out, both())
 
 
+@pytest.mark.gpu
 def test_plan_rule_and_workspace_bound():
     """Which calls are planned by length, and that a workspace sized for 64 equal splits covers them."""
     lib, bf = nat.lib(), nat.KVQ_BF16
@@ -158,6 +160,7 @@ def test_plan_rule_and_workspace_bound():
             assert n <= lib.kvq_decode_attn_workspace_bytes(B, Hq, Hkv, 1, 128, bf, bf, 64)
 
 
+@pytest.mark.gpu
 def test_workspace_of_the_equal_splits_is_still_enough():
     """A workspace that the caller sized for the library's equal splits: the
     call takes them, with the bytes of by_length = False."""
@@ -175,3 +178,100 @@ def test_workspace_of_the_equal_splits_is_still_enough():
     with ops.using_workspace(torch.zeros(max(size, 16), dtype=torch.uint8, device=DEV)):
         got = ops.decode_step(q, k, v, *cache, pos, **kw)
     assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_operators_split_equally_unless_asked():
+    """The operators' defaults over device lengths: equal splits, whose bits they have; by_length = True takes the
+    lengths' own, in every operator that has device lengths."""
+    B, Hq, Hkv, cap, G, P = 6, 32, 8, 16384, 32, 128
+    g = torch.Generator(device=DEV).manual_seed(17)
+    bufs = _cache(B, Hkv, cap, G, "bf16", g)
+    lens = _lengths("one_long", B, cap, g)
+    q = torch.randn(B, Hq, 1, 128, generator=g, device=DEV).bfloat16()
+    k, v = (torch.randn(B, Hkv, 1, 128, generator=g, device=DEV).bfloat16() for _ in range(2))
+    kw = dict(n_kv_heads=Hkv, group_size=G, sm_scale=128 ** -0.5)
+    n = nat.lib().kvq_decode_attn_num_splits(B, Hq, Hkv, 1, 128, cap, nat.KVQ_BF16, nat.KVQ_BF16, ops._num_cus(DEV))
+    pools = [t.transpose(0, 1).reshape(Hkv, B * cap, -1).contiguous() for t in bufs]
+    pt = ops.PageTable(torch.arange(B * cap // P, dtype=torch.int32, device=DEV).view(B, -1), P, B * cap // P)
+    calls = {
+        "step": lambda **o: ops.decode_step(q, k, v, *bufs, lens, **kw, **o),
+        "paged step": lambda **o: ops.decode_step_paged(q, k, v, *pools, pt, lens, **kw, **o),
+        "attention": lambda **o: ops.fused_decode_attention(q, *bufs, is_causal=False, seq_lens=lens, **kw, **o),
+        "paged attention": lambda **o: ops.fused_decode_attention_paged(q, *pools, pt, is_causal=False, seq_lens=lens,
+                                                                        **kw, **o),
+    }
+    for name, call in calls.items():
+        equal, dealt = call(n_split=n), call(n_split=BY_LENGTH)
+        assert not torch.equal(equal, dealt), name  # (the long sequence's sums are in another order)
+        assert torch.equal(call(), equal), name
+        assert torch.equal(call(by_length=True), dealt), name
+
+
+def test_when_splits_by_length_pay():
+    """The caches' rule: never for lengths alike, for few sequences' small spread, or where the kernel has no such
+    plan; for one long sequence among short ones."""
+    def pays(lens, cap, Hq=32, Hkv=8, D=128, dt=torch.bfloat16, sd=None):
+        return ops.by_length_pays(len(lens), Hq, Hkv, D, dt, sd or dt, cap, sum(lens), max(lens), 256)
+
+    for B in (1, 2, 8, 32, 64):
+        for cap in (4096, 16384, 32768):
+            for n in (0, 100, cap // 4, cap - 1):
+                assert not pays([n] * B, cap)
+    long32 = [16383] + [256] * 31
+    assert pays(long32, 16384) and pays(long32, 16384, dt=torch.float16) and pays([16000] + [300] * 7, 16384)
+    assert not pays(long32, 16384, D=64) and not pays(long32, 16384, dt=torch.float32)
+    assert not pays(long32, 16384, sd=torch.float16)
+    assert not pays([2047] + [128] * 31, 8192)          # 12.9 us equal, 19.1 by length
+    assert not pays([16383, 9000] * 16, 16384)          # half as long
+    assert not pays([16383] + [256] * 64, 16384)        # more sequences than the plan takes
+    assert not pays(long32, 16384, Hq=4, Hkv=8)
+
+
+def test_host_lengths_of_a_ragged_layer():
+    from kvint4.cache_base import _lag
+
+    assert _lag(torch.tensor([5, 9, 0]), 9) == (13, 0)
+    assert _lag(torch.tensor([5, 4, -3]), 9) == (18, 4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("paged", [False, True])
+def test_caches_choose_by_their_lengths(monkeypatch, paged):
+    """Caches whose host knows the lengths ask for splits by length where the rule says so, and no longer after an
+    edit that leaves them unknown."""
+    from kvint4.llama3.kv_cache import QuantizedKVCache
+    from kvint4.paged_cache import PagedQuantizedKVCache
+
+    B, Hkv, S, D, G = 8, 8, 16000, 128, 32
+    g = torch.Generator(device=DEV).manual_seed(3)
+    k, v = (torch.randn(B, Hkv, S, D, generator=g, device=DEV).bfloat16() for _ in range(2))
+    q = torch.randn(B, 32, 1, D, generator=g, device=DEV).bfloat16()
+    kn, vn = k[:, :, :1].contiguous(), v[:, :, :1].contiguous()
+    name = "decode_step_paged" if paged else "decode_step"
+    real, seen = getattr(ops, name), []
+    monkeypatch.setattr(ops, name, lambda *a, **kw: (seen.append(kw["by_length"]), real(*a, **kw))[1])
+
+    def step(cache):
+        assert cache.append_and_attend(q, kn, vn, 0, n_kv_heads=Hkv, scale=D ** -0.5) is not None
+        return seen[-1]
+
+    def make(lens):
+        cache = PagedQuantizedKVCache(group_size=G, page_size=128) if paged else QuantizedKVCache(group_size=G)
+        cache.load_ragged(k, v, 0, lens)
+        return cache
+
+    spread = torch.tensor([S] + [300] * 7, dtype=torch.int32)
+    cache = make(spread)
+    assert step(cache) and step(cache)
+    cache.crop(-1)
+    assert step(cache)
+    if paged:
+        cache.crop(400)
+        assert not step(cache)
+    else:
+        cache.crop(15990)
+        assert not step(cache)
+        assert not step(make(spread.to(DEV)))  # lengths that only the device knows
+    assert not step(make(torch.tensor([S, S - 900] * 4, dtype=torch.int32)))
+    assert not step(make(torch.full((B,), S, dtype=torch.int32)))
