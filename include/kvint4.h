@@ -154,8 +154,8 @@ int64_t kvq_decode_attn_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int6
  * kvq_decode_attn_num_splits is to be used instead (bf16/fp16 with D = 128, one
  * query position and 2 to 64 sequences are supported; short caches gain
  * nothing), and never more than kvq_decode_attn_workspace_bytes of 64 splits.
- * In any other call a large n_split means as many equal splits as the cap
- * allows, as before.
+ * In any other call, and for any other large value, n_split means as many
+ * equal splits as the cap allows.
  */
 #define KVQ_SPLIT_BY_LENGTH (1 << 30)
 int64_t kvq_decode_attn_by_length_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,

@@ -2853,7 +2853,7 @@ static int decode_attn_impl(const void* q, int q_dtype, const int64_t* q_strides
   }
   // splits by length, if asked for and the workspace holds them
   RaggedPlan rag = {0, 0, 0};
-  if (n_split >= KVQ_SPLIT_BY_LENGTH && seq_lens != nullptr && p.mfma) {
+  if (n_split == KVQ_SPLIT_BY_LENGTH && seq_lens != nullptr && p.mfma) {
     rag = ragged_plan(B, Hq, Hkv, Sq, D, q_dtype, scale_dtype);
     if (rag.items > 0 && (workspace == nullptr || workspace_bytes < rag.bytes)) rag.items = 0;
   }

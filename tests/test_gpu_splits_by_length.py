@@ -208,6 +208,20 @@ def test_operators_split_equally_unless_asked():
         assert torch.equal(call(by_length=True), dealt), name
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_split", [(1 << 30) + 1, (1 << 31) - 1, 1 << 40])
+def test_other_large_split_counts_are_equal_splits(n_split):
+    """A split count past the cap means the cap, 64 equal splits; only KVQ_SPLIT_BY_LENGTH itself asks for the list."""
+    B, Hq, Hkv, cap, G = 3, 32, 8, 16384, 32
+    g = torch.Generator(device=DEV).manual_seed(18)
+    bufs = _cache(B, Hkv, cap, G, "bf16", g)
+    lens = _lengths("one_long", B, cap, g)
+    q = torch.randn(B, Hq, 1, 128, generator=g, device=DEV).bfloat16()
+    kw = dict(n_kv_heads=Hkv, group_size=G, sm_scale=128 ** -0.5, is_causal=False, seq_lens=lens)
+    want = ops.fused_decode_attention(q, *bufs, n_split=64, **kw)
+    assert torch.equal(ops.fused_decode_attention(q, *bufs, n_split=n_split, **kw), want)
+
+
 def test_when_splits_by_length_pay():
     """The caches' rule: never for lengths alike, for few sequences' small spread, or where the kernel has no such
     plan; for one long sequence among short ones."""
