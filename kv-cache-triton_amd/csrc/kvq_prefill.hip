@@ -79,8 +79,8 @@ struct PrefillArgs {
   // equal share of its 64-key tiles and writes fp32 partials — unnormalised
   // O rows [D] and (running max, sum) — for prefill_merge_kernel
   int n_split;
-  float* ws_o;   // [unit][split][rows][D]
-  float* ws_ml;  // [unit][split][rows][2]
+  float* ws_o;   // [row block][unit][split][rows][D]
+  float* ws_ml;  // [row block][unit][split][rows][2]
   // staged route: operand images of the units u0 .. u0 + n_units - 1 (unit =
   // b * Hkv + kvh), `tiles` tiles of 16 D pieces of 16 bytes each
   uint4* img;
@@ -174,9 +174,9 @@ __device__ __attribute__((noinline)) void store_tile_direct(uint16_t* k_dst, uin
 // SIMD): one more register halves the occupancy. NW = waves per workgroup
 // (4, or 8 for D = 128 with two row blocks): the workgroup's threads share
 // the dequantize of each K/V tile, so eight waves (one workgroup per CU
-// instead of two of four) halve its VALU per wave. Long blocks come here only
-// where they are not staged (no workspace for it, or a head's images over
-// kStageBytes).
+// instead of two of four) halve its VALU per wave. Long blocks come here
+// where they are not staged (staging_pays; no workspace for it, or a head's
+// images over kStageBytes).
 template <int D, bool F16, bool S_F16, int RB, bool PAGED, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(RB == 2 ? 2 : 1)))
 void prefill_attn_kernel(const PrefillArgs a) {
@@ -1129,20 +1129,39 @@ struct StagedPlan {
 };
 
 constexpr int64_t kStageBytes = int64_t(256) << 20;
-// Where staging starts to pay: the images cost a launch and 32 bytes of
-// traffic per key and dim pair, once per unit, and every 128 rows save one
-// dequantization of them. Measured, staged against not (us; 8 KV heads, D =
-// 128): 2K keys 1024 rows 38.1 / 35.9, 2048 rows 44.8 / 50.4; 4K keys 512 rows
-// 37.9 / 37.4, 1024 rows 45.6 / 52; 16K keys 128 rows 44.2 / 37.9, 256 rows
-// 48.7 / 52, 2048 rows 161 / 274; 32 units, 1K keys, 512 rows 35.9 / 37.6.
+// Where staging pays: the images cost a launch and 32 bytes of traffic per key
+// and dim pair, once per unit, and every 128 rows save one dequantization of
+// them. Measured, staged / unstaged (us; GQA 4, causal, D = 128 unless stated):
+//  - 2^24 of units x rows x keys and 256 rows (512 at D = 64): 8 units, 2K keys,
+//    1024 rows 38.1 / 35.9, 2048 rows 44.8 / 50.4; 16K keys, 128 rows 44.2 /
+//    37.9, 256 rows 48.7 / 52; D = 64, 32 units, 3K keys, 256 rows 34.7 / 29.4.
+//  - 1024 keys: 100 units, 512 keys, 512 rows 42.7 / 34.3, 1280 keys 63 / 87; 50
+//    units of D = 64, 512 keys, 2048 rows 33.5 / 26.1. Blocks of 8192 rows pay
+//    over fewer (64 units, 128 keys 120 / 125; at D = 64 from 512 keys).
+//  - where the unstaged kernel, too, has a full device of its largest row blocks
+//    (2^16 of units x rows), from 1024 rows: 128 units, 2K keys, 512 rows 101 /
+//    87, 1024 rows 166 / 178.
+//  - where the last round of workgroups is not nearly empty: 75 units of D = 64,
+//    1024 rows (300 workgroups of 256 rows on 256 CUs), 1K keys 54 / 47.
+// Of 1202 shapes (8 to 200 units, 64 to 4096 keys, 256 to 16384 rows, both head
+// dims, GQA 1 and 4) three take longer inside these lines than they took before
+// there was staging, by 3 to 5 %; with the first line alone 78 did, by up to a
+// third.
 constexpr int64_t kStagedMinRows = 256;
 constexpr int64_t kStagedMinWork = int64_t(1) << 24;  // units * rows * keys
+constexpr int64_t kStagedMinKeys = 1024;
+
+bool staging_pays(int64_t units, int64_t rows, int64_t Sk, int64_t D) {
+  if (rows < (D == 64 ? 2 : 1) * kStagedMinRows || units * rows * Sk < kStagedMinWork) return false;
+  if (Sk < kStagedMinKeys) return rows >= 8192 && (D == 128 || Sk >= 512);
+  return rows >= 1024 || units * rows < 65536;
+}
 
 StagedPlan staged_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D) {
   StagedPlan p = {0, 1, 0, 0, 0, 0};
   const int64_t rows = Sq * (Hq / Hkv), units = B * Hkv, tiles = (Sk + kKeys - 1) / kKeys;
   p.img_bytes = tiles * D * 256;
-  if (rows < kStagedMinRows || units * rows * Sk < kStagedMinWork || tiles == 0 || p.img_bytes > kStageBytes) return p;
+  if (tiles == 0 || p.img_bytes > kStageBytes || !staging_pays(units, rows, Sk, D)) return p;
   p.group = std::min<int64_t>(std::min<int64_t>(units, 32768), kStageBytes / p.img_bytes);
   p.nw = p.group * ((rows + 255) / 256) >= 256 ? 8 : 4;
   p.row_blocks = (rows + 32 * p.nw - 1) / (32 * p.nw);
@@ -1158,6 +1177,9 @@ StagedPlan staged_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t S
     }
   }
   p.part_rows = p.n_split > 1 ? n_wg * p.n_split * 32 * p.nw : 0;
+  // workgroups of the rounds that run (of 5 slots at least 3)
+  const int64_t wgs = n_wg * p.n_split;
+  if (Sk >= kStagedMinKeys && wgs > slots && 5 * wgs < 3 * slots * ((wgs + slots - 1) / slots)) p.nw = 0;
   return p;
 }
 
