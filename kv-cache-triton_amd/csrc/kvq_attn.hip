@@ -2447,12 +2447,16 @@ static int64_t min_split_tokens(bool mfma, int64_t D) {
 // 78 / 68; 8 KV heads of 128, GQA 4, 1K keys, 32 positions 29.9 / 33.8, 64
 // positions 54 / 34.5). Up to 512 keys at D = 64, where the VALU kernel has
 // few splits, from 192 rows (512 keys: 8 positions 11.7 / 12.5, 16 positions
-// 15.0 / 12.4). A decode token (Sq = 1) stays on the VALU kernel, which also
+// 15.0 / 12.4). Past 4096 keys a GQA block of D = 64 has its chunks' keys from
+// L2 on the VALU kernel, and the line is at 2048 rows (8K keys, 12 query heads
+// of 4 KV heads: 3 x 32 positions 123 / 134, 128 positions 121 / 128, 3 x 64
+// positions 188 / 135; MHA, 3 x 32 positions 179 / 135). A decode token (Sq = 1) stays on the VALU kernel, which also
 // appends, and so does a call that asks for splits.
 static bool use_f32_block(int64_t bh, int64_t rows_total, int64_t Sq, int64_t D, int64_t s_max, int q_dtype,
                           int64_t n_split_req) {
   if (q_dtype != KVQ_F32 || Sq < 2 || n_split_req > 1) return false;
-  return bh * rows_total >= (D == 64 ? (s_max <= 512 ? 192 : 1024) : 1280);
+  const bool long_gqa = rows_total > Sq && s_max > 4096;
+  return bh * rows_total >= (D == 64 ? (s_max <= 512 ? 192 : (long_gqa ? 2048 : 1024)) : 1280);
 }
 
 // Split-K plan: enough splits that B * Hkv * row_chunks * n_split workgroups
