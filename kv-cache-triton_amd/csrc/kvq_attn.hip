@@ -129,13 +129,13 @@ struct AttnArgs {
   int64_t bt_stride;
   int bt_cols, n_blocks, page_shift;
   uint32_t pool_rows;
-  // splits by length (kernels instantiated with RAGGED): work items per
-  // (KV head, row chunk), workgroups of a round among them, sequences
-  int items, slots, batch;
   uint32_t* ws_cnt;  // [kCntUnits] arrival counters, kCntStride words apart
                      // (zero between calls)
   float* ws_ml;      // [n_units][n_split][ROWS][2]  (max, sum)
   float* ws_o;       // [n_units][n_split][ROWS][D]
+  // splits by length (kernels instantiated with RAGGED): work items per
+  // (KV head, row chunk), workgroups of a round among them, sequences
+  int items, slots, batch;
 #if defined(KVQ_PHASE_STAMPS)
   unsigned long long* stamps;  // phase stamps, or null
 #endif
