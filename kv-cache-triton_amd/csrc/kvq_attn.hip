@@ -382,6 +382,26 @@ __device__ __forceinline__ bool ragged_item(const AttnArgs& a, int item, int& b,
   return true;
 }
 
+// A unit's splits: its part of the item list in a RAGGED launch. The other
+// launches' come from the arguments where they are needed: held from the start
+// of the kernel they cost the paged fp16 kernel of two row sets at D = 64 79
+// more spilled scalar registers (12 heads, 8 query positions over 1K keys, 8.9
+// -> 10.0 us; over 16K keys, 16 sequences, 77 -> 86).
+struct Parts {
+  int ns;         // splits of the unit
+  int64_t first;  // its first partial slot
+};
+template <bool RAGGED>
+__device__ __forceinline__ int parts_ns(const AttnArgs& a, const Parts& p) {
+  if constexpr (RAGGED) return p.ns;
+  else return a.n_split;
+}
+template <bool RAGGED>
+__device__ __forceinline__ int64_t parts_first(const AttnArgs& a, const Parts& p, int unit) {
+  if constexpr (RAGGED) return p.first;
+  else return (int64_t)unit * a.n_split;
+}
+
 __device__ __forceinline__ int64_t out_index(const AttnArgs& a, int b, int kvh, int rho, int d) {
   const int hq = (int)fdiv((uint32_t)rho, a.div_sq), qi = rho - hq * a.Sq;
   const int head = kvh * a.ratio + hq;
@@ -546,8 +566,8 @@ __device__ __forceinline__ float group_reduce(float v) {
 // barrier after the last load), and the lanes of group 0 store the 4
 // outputs of their pieces. A row no split saw a key for (all l_s = 0) yields
 // zeros.
-template <int ROWS, int D, int OUT_DT, int NW>
-__device__ __forceinline__ void merge_splits(const AttnArgs& a, int64_t part0, int ns, int rc, int kvh, int b,
+template <int ROWS, int D, int OUT_DT, int NW, bool RAGGED>
+__device__ __forceinline__ void merge_splits(const AttnArgs& a, int unit, const Parts& parts, int rc, int kvh, int b,
                                              MergeLds& mg) {
   constexpr int NT = 64 * NW;
   constexpr int Q = ROWS * D / 4;  // 16-byte pieces per split
@@ -558,10 +578,11 @@ __device__ __forceinline__ void merge_splits(const AttnArgs& a, int64_t part0, i
   constexpr int MLPT = (kMaxSplit * kMaxRows + NT - 1) / NT;  // (max, sum) loads per thread
   constexpr int PW = 64 / P;       // pieces per wave
   const int tid = threadIdx.x;
+  const int ns = parts_ns<RAGGED>(a, parts);
   const int lane = tid & 63;
   const int piece = (tid >> 6) * PW + lane % PW, grp = lane / PW;
   const int r = piece / (D / 4), d4 = piece % (D / 4);
-  const int64_t slot0 = part0 * ROWS;  // + split * ROWS + row
+  const int64_t slot0 = parts_first<RAGGED>(a, parts, unit) * ROWS;  // + split * ROWS + row
   const __amdgpu_buffer_rsrc_t ro =
       buffer_rsrc(a.ws_o + slot0 * D, (uint32_t)((int64_t)ns * ROWS * D * 4));
   const __amdgpu_buffer_rsrc_t rm = buffer_rsrc(a.ws_ml + slot0 * 2, (uint32_t)(ns * ROWS * 8));
@@ -663,16 +684,16 @@ __device__ __forceinline__ void merge_splits(const AttnArgs& a, int64_t part0, i
 // row it is masked from) and its values at nt[ROWS + d], the same for every
 // row. The MFMA kernel's decode step passes the new token this way.
 //
-// The unit has ns splits, whose partials are slots part0 .. part0 + ns - 1 of
-// the workspace.
-template <int ROWS, int D, int OUT_DT, int NW>
-__device__ __forceinline__ void finish_block(const AttnArgs& a, int unit, int split, int ns, int64_t part0, int rc,
+// The partials of the unit's splits are the workspace's slots from
+// parts_first on.
+template <int ROWS, int D, int OUT_DT, int NW, bool RAGGED>
+__device__ __forceinline__ void finish_block(const AttnArgs& a, int unit, int split, const Parts& parts, int rc,
                                              int kvh, int b, const float (*o_lds)[ROWS][D],
                                              const float (*ml_lds)[ROWS][2], MergeLds& mg,
                                              const float* nt = nullptr) {
   constexpr int NT = 64 * NW;
   const int tid = threadIdx.x;
-  const bool single = ns == 1;
+  const bool single = parts_ns<RAGGED>(a, parts) == 1;
   for (int idx = tid; idx < ROWS * D; idx += NT) {
     const int r = idx / D, d = idx % D;
     float mw[NW], lw[NW];
@@ -703,7 +724,7 @@ __device__ __forceinline__ void finish_block(const AttnArgs& a, int unit, int sp
       if (rho < a.rows_total)
         store_from_f32(a.out, out_index(a, b, kvh, rho, d), OUT_DT, Ls > 0.0f ? Os / Ls : 0.0f);
     } else {
-      const int64_t slot = (part0 + split) * ROWS + r;
+      const int64_t slot = (parts_first<RAGGED>(a, parts, unit) + split) * ROWS + r;
       a.ws_o[slot * D + d] = Os;
       if (d == 0) *(float2*)&a.ws_ml[slot * 2] = make_float2(M, Ls);
     }
@@ -716,12 +737,12 @@ __device__ __forceinline__ void finish_block(const AttnArgs& a, int unit, int sp
   uint32_t* cnt = a.ws_cnt + (int64_t)unit * kCntStride;
   if (tid == 0)
     mg.last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-              (uint32_t)(ns - 1);
+              (uint32_t)(parts_ns<RAGGED>(a, parts) - 1);
     KVQ_STAMP(7);
   __syncthreads();
   if (!mg.last) return;
   KVQ_STAMP(8);
-  merge_splits<ROWS, D, OUT_DT, NW>(a, part0, ns, rc, kvh, b, mg);
+  merge_splits<ROWS, D, OUT_DT, NW, RAGGED>(a, unit, parts, rc, kvh, b, mg);
   if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -897,21 +918,19 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
   // into waits for it too).
   asm volatile("" ::"s"(a.bt_cols), "s"(a.ws_o));
   int unit, split, b, kvh, rc;
-  int ns, split_keys = 0, L;  // the unit's splits; (RAGGED) keys of a split; the sequence's length
-  int64_t part0;              // the unit's first partial slot
+  int split_keys = 0, L;  // (RAGGED) keys of a split; the sequence's length
+  Parts parts;            // (RAGGED)
   if constexpr (RAGGED) {
     const int hc = (int)((blockIdx.x & 7u) + 8u * blockIdx.y);
     int first;
-    if (hc >= a.Hkv * a.row_chunks || !ragged_item(a, (int)(blockIdx.x >> 3), b, split, ns, first, split_keys, L))
+    if (hc >= a.Hkv * a.row_chunks || !ragged_item(a, (int)(blockIdx.x >> 3), b, split, parts.ns, first, split_keys, L))
       return;
     kvh = (int)fdiv((uint32_t)hc, a.div_rc);
     rc = hc - kvh * a.row_chunks;
     unit = (b * a.Hkv + kvh) * a.row_chunks + rc;
-    part0 = (int64_t)hc * a.items + first;
+    parts.first = (int64_t)hc * a.items + first;
   } else {
     if (!unit_and_split(a, unit, split)) return;
-    ns = a.n_split;
-    part0 = (int64_t)unit * ns;
   }
   // The two waves of a SIMD (w and w + 4) run the same scalar prologue, and a
   // SIMD issues one scalar instruction per turn: raising the first one's
@@ -925,7 +944,7 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
   // 9.33 -> 9.26 us, C2 7.27 -> 7.29 us; with four waves per SIMD, C5 lost
   // 0.28 us that way).
   {
-    const bool app = D == 128 && RS == 1 && a.append && split == ns - 1 && (wave % (NW / 2)) >= NW / 2 - 2;
+    const bool app = D == 128 && RS == 1 && a.append && split == parts_ns<RAGGED>(a, parts) - 1 && (wave % (NW / 2)) >= NW / 2 - 2;
     if ((wave < NW / 2) != app) __builtin_amdgcn_s_setprio(1);
   }
   if constexpr (!RAGGED) {
@@ -968,7 +987,7 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
   L = L < 0 ? 0 : L;
   // decode step: the new token goes to row L (if it fits the cache) and is
   // attended by the unit's last split from registers
-  bool has_new = a.append && len_ok && L < a.Sk && split == ns - 1;
+  bool has_new = a.append && len_ok && L < a.Sk && split == parts_ns<RAGGED>(a, parts) - 1;
   L = L < a.Sk ? L : a.Sk;
   // The new token's rows (lane l: elements 2l, 2l+1): the K row for the
   // split's last wave, which quantizes, stores and scores it, the V row for
@@ -1702,7 +1721,8 @@ void decode_attn_mfma_kernel(const AttnArgs a) {
   __syncthreads();
   // the new token (scores and values in LDS, written by the K and V waves
   // before their tile loops) joins the waves' partials in the workgroup fold
-  finish_block<ROWS, D, QM, NW>(a, unit, split, ns, part0, rc, kvh, b, o_lds, ml_lds, mg, has_new ? nt_lds : nullptr);
+  finish_block<ROWS, D, QM, NW, RAGGED>(a, unit, split, parts, rc, kvh, b, o_lds, ml_lds, mg,
+                                        has_new ? nt_lds : nullptr);
   KVQ_STAMP(11);
 }
 
@@ -2406,8 +2426,8 @@ __global__ __launch_bounds__(256) void decode_attn_valu_kernel(const AttnArgs a)
   __syncthreads();
   // the new token (scores and values in LDS, written by waves 3 and 2 before
   // their tile loops) joins the waves' partials in the workgroup fold
-  finish_block<ROWS, D, QM, 4>(a, unit, split, a.n_split, (int64_t)unit * a.n_split, rc, kvh, b, o_lds, ml_lds, mg,
-                               has_new ? nt_lds : nullptr);
+  finish_block<ROWS, D, QM, 4, false>(a, unit, split, Parts{}, rc, kvh, b, o_lds, ml_lds, mg,
+                                      has_new ? nt_lds : nullptr);
 }
 
 // ---------------------------------------------------------------------------
