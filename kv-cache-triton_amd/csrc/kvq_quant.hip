@@ -44,10 +44,18 @@ struct QuantArgs {
 // One launch quantizes one tensor, or a layer's K and V together (blockIdx.y
 // picks the tensor): an append is then one launch instead of two. A 16K
 // prompt's K and V ([1, 8, 16384, 128] bf16 each, strided as a projection
-// leaves them): 2 x 12.6 us as two launches, 21.1 us as one (4.1 TB/s).
-struct QuantPair {
-  QuantArgs t[2];
+// leaves them): 2 x 12.6 us as two launches, 21.1 us as one (4.1 TB/s). A launch
+// of one tensor has an argument block of its own: choosing among two costs a
+// small one 0.15 us of 2.6 (one token of 16 sequences).
+template <int N>
+struct QuantArgsOf {
+  QuantArgs t[N];
 };
+template <int N>
+__device__ __forceinline__ const QuantArgs& own_args(const QuantArgsOf<N>& p) {
+  if constexpr (N == 1) return p.t[0];
+  else return p.t[blockIdx.y];
+}
 
 // Destination row of (b, position), or -1 where it does not exist: the
 // position itself in the contiguous layout (if inside [0, cap)), its pool row
@@ -63,9 +71,9 @@ __device__ __forceinline__ float ld_x(const void* p, int64_t i) {
   else return ((const float*)p)[i];
 }
 
-template <int XDT>
-__global__ __launch_bounds__(256) void quantize_kernel(const QuantPair p) {
-  const QuantArgs& a = p.t[blockIdx.y];
+template <int XDT, int N>
+__global__ __launch_bounds__(256) void quantize_kernel(const QuantArgsOf<N> p) {
+  const QuantArgs& a = own_args(p);
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= a.rows * a.ngroups) return;
   const int64_t row = idx / a.ngroups;
@@ -156,9 +164,9 @@ constexpr int64_t kSmallChunks = 256 * 1024;
 // LPG = lanes per group = G / 8. PAD: D is no multiple of G, so the last group
 // has chunks of padding (their selects cost the others 4 %: [2, 32, 3001, 128]
 // bf16, G = 32, 16.6 us without, 17.4 with).
-template <int XDT, int LPG, int RPT, bool PAD>
-__global__ __launch_bounds__(256) void quantize_vec_kernel(const QuantPair p) {
-  const QuantArgs& a = p.t[blockIdx.y];
+template <int XDT, int LPG, int RPT, bool PAD, int N>
+__global__ __launch_bounds__(256) void quantize_vec_kernel(const QuantArgsOf<N> p) {
+  const QuantArgs& a = own_args(p);
   const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t cpr = a.cpr;  // chunks per padded row (ngroups * G / 8)
   const uint32_t rows = (uint32_t)a.rows;
@@ -431,21 +439,34 @@ using namespace kvq;
 
 namespace {
 
-template <int XDT, int RPT, bool PAD>
-void launch_qvec_pad(int lpg, dim3 grid, hipStream_t st, const QuantPair& a) {
+template <int XDT, int RPT, bool PAD, int N>
+void launch_qvec_pad(int lpg, dim3 grid, hipStream_t st, const QuantArgsOf<N>& a) {
   switch (lpg) {
-    case 1: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 1, RPT, PAD>), grid, dim3(256), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 2, RPT, PAD>), grid, dim3(256), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 4, RPT, PAD>), grid, dim3(256), 0, st, a); break;
-    case 8: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 8, RPT, PAD>), grid, dim3(256), 0, st, a); break;
-    default: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 16, RPT, PAD>), grid, dim3(256), 0, st, a); break;
+    case 1: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 1, RPT, PAD, N>), grid, dim3(256), 0, st, a); break;
+    case 2: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 2, RPT, PAD, N>), grid, dim3(256), 0, st, a); break;
+    case 4: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 4, RPT, PAD, N>), grid, dim3(256), 0, st, a); break;
+    case 8: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 8, RPT, PAD, N>), grid, dim3(256), 0, st, a); break;
+    default: hipLaunchKernelGGL((quantize_vec_kernel<XDT, 16, RPT, PAD, N>), grid, dim3(256), 0, st, a); break;
   }
 }
 
-template <int XDT, int RPT>
-void launch_qvec(bool pad, int lpg, dim3 grid, hipStream_t st, const QuantPair& a) {
-  if (pad) launch_qvec_pad<XDT, RPT, true>(lpg, grid, st, a);
-  else launch_qvec_pad<XDT, RPT, false>(lpg, grid, st, a);
+template <int XDT, int N>
+void launch_quant(bool vec, bool small, bool pad, int lpg, dim3 grid, hipStream_t st, const QuantArgsOf<N>& a) {
+  if (!vec) hipLaunchKernelGGL((quantize_kernel<XDT, N>), grid, dim3(256), 0, st, a);
+  else if (small && pad) launch_qvec_pad<XDT, 1, true>(lpg, grid, st, a);
+  else if (small) launch_qvec_pad<XDT, 1, false>(lpg, grid, st, a);
+  else if (pad) launch_qvec_pad<XDT, kQuantRows, true>(lpg, grid, st, a);
+  else launch_qvec_pad<XDT, kQuantRows, false>(lpg, grid, st, a);
+}
+
+template <int N>
+void launch_quant_dtype(int x_dtype, bool vec, bool small, bool pad, int lpg, dim3 grid, hipStream_t st,
+                        const QuantArgsOf<N>& a) {
+  switch (x_dtype) {
+    case KVQ_BF16: launch_quant<KVQ_BF16>(vec, small, pad, lpg, grid, st, a); break;
+    case KVQ_F16: launch_quant<KVQ_F16>(vec, small, pad, lpg, grid, st, a); break;
+    default: launch_quant<KVQ_F32>(vec, small, pad, lpg, grid, st, a); break;
+  }
 }
 
 template <int ODT, int RPT>
@@ -516,7 +537,7 @@ int quantize_impl(const char* who, int n, const QuantTensor* t, int x_dtype,
   const bool vec_shape = group_size % 8 == 0 && group_size <= 128 && (lpg & (lpg - 1)) == 0 && D % 8 == 0 &&
                          rows * cpr < (1ll << 32) - 256 * kQuantRows;
   bool vec_t[2] = {vec_shape, vec_shape};
-  QuantPair p;
+  QuantArgsOf<2> p;
   for (int i = 0; i < 2; ++i) {
     const QuantTensor& u = t[i < n ? i : 0];
     QuantArgs& a = p.t[i];
@@ -548,31 +569,13 @@ int quantize_impl(const char* who, int n, const QuantTensor* t, int x_dtype,
     }
     return KVQ_OK;
   }
-  const bool vec = vec_t[0];
-  hipStream_t st = (hipStream_t)stream;
-  if (vec) {
-    const bool small = n * rows * cpr <= kSmallChunks;
-    const bool pad = D % group_size != 0;
-    const int rpt = small ? 1 : kQuantRows;
-    const int64_t total = (rows + rpt - 1) / rpt * cpr;
-    const dim3 grid((unsigned)((total + 255) / 256), (unsigned)n);
-    switch (x_dtype) {
-      case KVQ_BF16: small ? launch_qvec<KVQ_BF16, 1>(pad, lpg, grid, st, p) : launch_qvec<KVQ_BF16, kQuantRows>(pad, lpg, grid, st, p); break;
-      case KVQ_F16: small ? launch_qvec<KVQ_F16, 1>(pad, lpg, grid, st, p) : launch_qvec<KVQ_F16, kQuantRows>(pad, lpg, grid, st, p); break;
-      default: small ? launch_qvec<KVQ_F32, 1>(pad, lpg, grid, st, p) : launch_qvec<KVQ_F32, kQuantRows>(pad, lpg, grid, st, p); break;
-    }
-    KVQ_CHECK_LAUNCH(who);
-    return KVQ_OK;
-  }
-
-  const int64_t total = rows * ngroups;
-  const dim3 block(256);
+  const bool vec = vec_t[0], small = n * rows * cpr <= kSmallChunks, pad = D % group_size != 0;
+  const int64_t rpt = small ? 1 : kQuantRows;
+  const int64_t total = vec ? (rows + rpt - 1) / rpt * cpr : rows * ngroups;
   const dim3 grid((unsigned)((total + 255) / 256), (unsigned)n);
-  switch (x_dtype) {
-    case KVQ_BF16: hipLaunchKernelGGL(quantize_kernel<KVQ_BF16>, grid, block, 0, st, p); break;
-    case KVQ_F16: hipLaunchKernelGGL(quantize_kernel<KVQ_F16>, grid, block, 0, st, p); break;
-    default: hipLaunchKernelGGL(quantize_kernel<KVQ_F32>, grid, block, 0, st, p); break;
-  }
+  hipStream_t st = (hipStream_t)stream;
+  if (n == 1) launch_quant_dtype(x_dtype, vec, small, pad, lpg, grid, st, QuantArgsOf<1>{{p.t[0]}});
+  else launch_quant_dtype(x_dtype, vec, small, pad, lpg, grid, st, p);
   KVQ_CHECK_LAUNCH(who);
   return KVQ_OK;
 }
