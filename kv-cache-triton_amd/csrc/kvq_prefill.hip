@@ -1141,12 +1141,15 @@ constexpr int64_t kStageBytes = int64_t(256) << 20;
 //  - where the unstaged kernel, too, has a full device of its largest row blocks
 //    (2^16 of units x rows), from 1024 rows: 128 units, 2K keys, 512 rows 101 /
 //    87, 1024 rows 166 / 178.
+//  - images of all units under 64 MiB, above that from 512 rows, past kStageBytes
+//    (units then go in groups, and the images through memory) from 2048 rows,
+//    1024 at D = 64: 32 units, 4K keys, 256 rows 56 / 50; 128 units, 16K keys, 256
+//    rows 611 / 403, 1024 rows 1301 / 1199, 2048 rows 2051 / 2297.
 //  - where the last round of workgroups is not nearly empty: 75 units of D = 64,
 //    1024 rows (300 workgroups of 256 rows on 256 CUs), 1K keys 54 / 47.
-// Of 1202 shapes (8 to 200 units, 64 to 4096 keys, 256 to 16384 rows, both head
-// dims, GQA 1 and 4) three take longer inside these lines than they took before
-// there was staging, by 3 to 5 %; with the first line alone 78 did, by up to a
-// third.
+// Of 2014 shapes (8 to 200 units, 64 to 32K keys, 256 to 16384 rows, both head
+// dims, GQA 1 and 4) sixteen take longer inside these lines than without
+// staging, by 2 to 14 %; with the first line alone 140 did, by up to 42 %.
 constexpr int64_t kStagedMinRows = 256;
 constexpr int64_t kStagedMinWork = int64_t(1) << 24;  // units * rows * keys
 constexpr int64_t kStagedMinKeys = 1024;
@@ -1154,6 +1157,9 @@ constexpr int64_t kStagedMinKeys = 1024;
 bool staging_pays(int64_t units, int64_t rows, int64_t Sk, int64_t D) {
   if (rows < (D == 64 ? 2 : 1) * kStagedMinRows || units * rows * Sk < kStagedMinWork) return false;
   if (Sk < kStagedMinKeys) return rows >= 8192 && (D == 128 || Sk >= 512);
+  const int64_t images = units * ((Sk + kKeys - 1) / kKeys) * D * 256;
+  if (images > kStageBytes) return rows >= (D == 64 ? 1024 : 2048);
+  if (images >= kStageBytes / 4 && rows < 512) return false;
   return rows >= 1024 || units * rows < 65536;
 }
 

@@ -228,3 +228,18 @@ def test_staged_largest_scales():
     assert ks.float().max().item() > 2.0 ** 125
     want = _want(q, _dequant64(kp, ks, G, D), _dequant64(vp, vs, G, D), 8e-30, True)
     _compare(q, kp, ks, vp, vs, Hkv, G, True, 8e-30, want)
+
+
+def test_staged_long_blocks_in_groups():
+    """Units in groups (31 and 9 of 40) with eight waves per workgroup: 2048 rows over 16448 keys."""
+    B, Hq, Hkv, Sq, Sk, D, G = 5, 32, 8, 512, 16448, 128, 32
+    g = torch.Generator(device=DEV).manual_seed(13)
+    shape = (B, Hq, Hkv, Sq, D, Sk)
+    n = nat.lib().kvq_prefill_attn_staged_workspace_bytes(*shape)
+    assert (200 << 20) < n < (320 << 20) and n > nat.lib().kvq_prefill_attn_workspace_bytes(*shape)
+    q = torch.randn(B, Hq, Sq, D, generator=g, device=DEV).to(torch.bfloat16)
+    kp, ks, vp, vs = _quantized(B, Hkv, Sk, D, "bf16", G, g)
+    a = _call(q, kp, ks, vp, vs, Hkv, G, True, D ** -0.5, True)
+    b = _call(q, kp, ks, vp, vs, Hkv, G, True, D ** -0.5, False)
+    # outputs average thousands of values (|out| < 0.2): two bf16 roundings of them and of the weights
+    assert (a.float() - b.float()).abs().max().item() <= 2e-3

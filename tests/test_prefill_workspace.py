@@ -33,7 +33,7 @@ def test_no_room_for_images_takes_the_unstaged_scratch(monkeypatch, Sq, Sk):
 @pytest.mark.parametrize("units,rows,Sk,D,staged", [
     (8, 2048, 1024, 128, True),       # 2^24 of units x rows x keys
     (8, 2047, 1024, 128, False),
-    (32, 256, 4096, 128, True),       # 256 rows, 512 at D = 64
+    (31, 256, 4096, 128, True),       # 256 rows, 512 at D = 64
     (64, 255, 4096, 128, False),
     (32, 512, 4096, 64, True),
     (64, 511, 4096, 64, False),
@@ -43,6 +43,12 @@ def test_no_room_for_images_takes_the_unstaged_scratch(monkeypatch, Sq, Sk):
     (127, 512, 2048, 128, True),      # a full device of the unstaged kernel's 256-row blocks: from 1024 rows
     (128, 512, 2048, 128, False),
     (128, 1024, 2048, 128, True),
+    (32, 256, 4096, 128, False),      # 64 MiB of images: from 512 rows
+    (32, 512, 4096, 128, True),
+    (40, 2047, 16448, 128, False),    # more than 256 MiB: from 2048 rows, 1024 at D = 64
+    (40, 2048, 16448, 128, True),
+    (80, 1023, 16448, 64, False),
+    (80, 1024, 16448, 64, True),
     (75, 1024, 1024, 64, False),      # 300 workgroups on 256 CUs
     (80, 1024, 1024, 64, True),       # 320: the second round a quarter full
 ])
