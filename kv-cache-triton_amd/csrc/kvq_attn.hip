@@ -316,15 +316,18 @@ __device__ __forceinline__ int ceil_div(int n, int w, float inv) {
 // Splits by length: a batch of very different lengths (device lengths, at
 // most 64 sequences, one per lane). With one split count for all, the longest
 // sequence's workgroups outlast the rest (a paged batch of 32 sequences of 256
-// to 16K keys, one split each: 66 us, of which the bytes need 28; 38 us by length). Here every split holds W
-// keys, sequence b has ns_b = max(1, ceil(L_b / W)) of them, and the launch's
+// to 16K keys, one split each: 66 us, of which the bytes need 28; 36 to 43 us
+// by length, by the drawn lengths). Here every split holds W keys, sequence b
+// has ns_b = max(1, ceil(L_b / W)) of them, and the launch's
 // workgroups are items of one list per (KV head, row chunk): sequence 0's
 // splits, sequence 1's, ... Every wave works the list out from the lengths,
 // lane b holding sequence b's.
 // W = the longest length / k, for the k of a table whose estimate is the
 // shortest: with all items in one round of resident workgroups W + A keys,
 // else the average (T + A items) / slots plus half of that; A = 1200 keys
-// stands for a workgroup's prologue, fold and merge. The estimates count items
+// stands for a workgroup's prologue, fold and merge (32 sequences of up to 16K
+// keys 31.3 us; with A = 600 32.9, 2400 32.6; 24 sequences 30.0, 30.2, 31.4; up
+// to 20 sequences, one round, alike). The estimates count items
 // in floats; if the exact count of the chosen W does not fit the list, W is
 // the longest length (one item per sequence, which the host leaves room for).
 // Item -> (b, split, ns, first item of b, W); false: no such item.
@@ -2538,7 +2541,11 @@ static int64_t workspace_bytes_for(const Plan& p, int64_t D) {
 // Splits by length (RAGGED kernels): D = 128, one query position, matching
 // 16-bit types, 2 to 64 sequences. Items per (KV head, row chunk): one round
 // of workgroups (a CU holds one) for up to 5/8 as many sequences, two for up
-// to 3/2, a round more than the sequences need beyond. Workgroups whose item
+// to 3/2, a round more than the sequences need beyond (8 KV heads, 32
+// workgroups a round, lengths of 256 to 16K keys, us: 20 sequences in one round
+// 25.4, in two 25.8; 24 in two 30.0, in one 32.6; 28 30.2 and 40.9; 40 in two
+// 41.2, in three 39.3; 48 45.2 and 44.4; 56 in three 45.4, in two 49.5; 64 55.5
+// and 84.3). Workgroups whose item
 // does not exist exit after working out the list, but in a launch of more than
 // one round they do that behind the others (about 2 us), so rounds are not
 // added freely. The partials are slots of the items, so the

@@ -2,19 +2,21 @@
  * kvq_pyhost.c — the CPython side of the hot operators: calls into
  * libkvint4.so (include/kvint4.h) with arguments taken straight from tensors.
  *
- * A decode step is a 9 us launch whose C entry point takes 38 arguments. Built
- * up through ctypes (an array object per stride list, a conversion per
- * argument) an eager step of the cache class cost the host 18.8 us; through
- * this module it costs 9.6, and a prompt's append 21 instead of 34.
+ * A decode step is a 9 us launch whose C entry point takes 31 arguments (35
+ * over a paged cache). Built up through ctypes (an array object per stride
+ * list, a conversion per argument) an eager step of the cache class cost the
+ * host 18.8 us; through this module it costs 9.6, and a prompt's append 21
+ * instead of 34.
  *
  * Conventions of every function below: positional arguments; a tensor argument
  * is a torch tensor (its data_ptr() and stride() are called), a tuple
  * (pointer, strides) where the caller views it under other strides, or None
  * (a null pointer); plain pointers are integers or None; the result is the C
  * entry point's status (kvint4._native.check turns it into an exception, with
- * kvq_last_error() of the same thread). The checks that a caller relies on are
- * the Python operator's and the C entry point's. The GIL is released around
- * the launch, as ctypes does.
+ * kvq_last_error() of the same thread). Checked here are the number of
+ * arguments and their types; the checks of values that a caller relies on are
+ * the Python operator's and the C entry point's. The GIL is released around the
+ * launch, as ctypes does.
  */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>

@@ -144,3 +144,7 @@ def build(verbose: bool = False) -> str:
                 verbose)
     _build_host(verbose)
     return OUT
+
+
+if __name__ == "__main__":
+    build(verbose=True)
