@@ -9,12 +9,12 @@
  * instead of 34.
  *
  * Conventions of every function below: positional arguments; a tensor argument
- * is a torch tensor (its data_ptr() and stride() are called), a tuple
+ * is a torch tensor on the GPU (data_ptr() and stride() are called), a tuple
  * (pointer, strides) where the caller views it under other strides, or None
  * (a null pointer); plain pointers are integers or None; the result is the C
  * entry point's status (kvint4._native.check turns it into an exception, with
  * kvq_last_error() of the same thread). Checked here are the number of
- * arguments and their types; the checks of values that a caller relies on are
+ * arguments, their types and the tensors' device; the checks of values that a caller relies on are
  * the Python operator's and the C entry point's. The GIL is released around the
  * launch, as ctypes does.
  */
@@ -25,7 +25,7 @@
 
 #include "../../include/kvint4.h"
 
-static PyObject *s_data_ptr, *s_stride;
+static PyObject *s_data_ptr, *s_stride, *s_is_cuda, *s_is_pinned;
 
 typedef struct {
   void *p;
@@ -71,6 +71,19 @@ static int read_tensor(PyObject *o, tensor_arg *a, Py_ssize_t n) {
   const int rp = read_pointer(p, &a->p);
   Py_DECREF(p);
   if (rp < 0) return -1;
+  /* a host pointer would fault the GPU at the kernel's first read (pinned memory, which it can read, does not) */
+  PyObject *gpu = PyObject_GetAttr(o, s_is_cuda);
+  if (gpu != NULL && gpu != Py_True) {
+    Py_DECREF(gpu);
+    gpu = PyObject_CallMethodNoArgs(o, s_is_pinned);
+  }
+  if (gpu == NULL) return -1;
+  const int reachable = gpu == Py_True;
+  Py_DECREF(gpu);
+  if (!reachable) {
+    PyErr_SetString(PyExc_ValueError, "expected GPU tensors (got one in host memory)");
+    return -1;
+  }
   PyObject *st = PyObject_CallMethodNoArgs(o, s_stride);
   if (st == NULL) return -1;
   const int rs = read_strides(st, a->st, n);
@@ -414,6 +427,8 @@ static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_kvq_host", "libkvin
 PyMODINIT_FUNC PyInit__kvq_host(void) {
   s_data_ptr = PyUnicode_InternFromString("data_ptr");
   s_stride = PyUnicode_InternFromString("stride");
-  if (s_data_ptr == NULL || s_stride == NULL) return NULL;
+  s_is_cuda = PyUnicode_InternFromString("is_cuda");
+  s_is_pinned = PyUnicode_InternFromString("is_pinned");
+  if (s_data_ptr == NULL || s_stride == NULL || s_is_cuda == NULL || s_is_pinned == NULL) return NULL;
   return PyModule_Create(&module);
 }

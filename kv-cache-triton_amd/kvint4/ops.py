@@ -429,8 +429,6 @@ def fused_decode_attention(
     it does not handle. q [B, Hq, Sq, D]; K/V codes [B, Hkv, Sk, W] (strided views
     of a larger cache are fine as long as the last dim is contiguous).
     `n_split` overrides the planner's sequence-split count (tuning)."""
-    _check_cuda(q, k_packed, k_scales, v_packed, v_scales, *(() if out is None else (out,)),
-                what="fused_decode_attention")
     B, Hq, Sq, D = q.shape
     Sk = k_packed.shape[2]
     if out is None:
@@ -479,7 +477,6 @@ def prefill_attention(
     matrix cores (kvq_prefill_attn); raises KVQUnsupported for shapes or
     dtypes it does not handle. q [B, Hq, Sq, D]; K/V codes [B, Hkv, Sk, W],
     one length Sk for the batch; causal masking aligned bottom-right."""
-    _check_cuda(q, k_packed, k_scales, v_packed, v_scales, *(() if out is None else (out,)), what="prefill_attention")
     B, Hq, Sq, D = q.shape
     Sk = k_packed.shape[2]
     if q.stride(-1) != 1:
@@ -531,8 +528,6 @@ def decode_step(
     `by_length` = True, for device positions that differ a lot
     (by_length_pays): the splits are dealt to the sequences by their lengths
     instead of the same number to each."""
-    _check_cuda(q, k_new, v_new, k_packed, k_scales, v_packed, v_scales, *(() if out is None else (out,)),
-                what="decode_step")
     B, Hq, Sq, D = q.shape
     if Sq != 1:
         raise nat.KVQUnsupported("decode_step handles one query position")
@@ -887,8 +882,7 @@ def fused_decode_attention_paged(
     queries with 16-bit scales run on the matrix cores, fp32 queries or scales
     on the exact-fp32 kernel. Raises KVQUnsupported where neither applies
     (page_size < 64)."""
-    _check_cuda(q, k_pool, k_scales, v_pool, v_scales, pt.table, *(() if out is None else (out,)),
-                what="fused_decode_attention_paged")
+    _check_cuda(q, k_pool, k_scales, v_pool, v_scales, pt.table, what="fused_decode_attention_paged")
     B, Hq, Sq, D = q.shape
     if pt.table.shape[0] < B:
         raise ValueError("block table has fewer rows than the batch")
@@ -939,8 +933,7 @@ def prefill_attention_paged(
     """prefill_attention over a paged cache: every sequence attends its first
     seq_len tokens through the block table (pages of >= 64 rows); raises
     KVQUnsupported for shapes or dtypes the kernel does not handle."""
-    _check_cuda(q, k_pool, k_scales, v_pool, v_scales, pt.table, *(() if out is None else (out,)),
-                what="prefill_attention_paged")
+    _check_cuda(q, k_pool, v_pool, pt.table, what="prefill_attention_paged")
     B, Hq, Sq, D = q.shape
     if pt.table.shape[0] < B:
         raise ValueError("block table has fewer rows than the batch")
@@ -987,8 +980,7 @@ def decode_step_paged(
     position (int, or device int32 [B] of old lengths) through the block table;
     a position whose page has no block is neither written nor attended.
     `by_length` as for decode_step."""
-    _check_cuda(q, k_new, v_new, k_pool, k_scales, v_pool, v_scales, pt.table, *(() if out is None else (out,)),
-                what="decode_step_paged")
+    _check_cuda(q, k_new, v_new, k_pool, pt.table, what="decode_step_paged")
     B, Hq, Sq, D = q.shape
     if pt.table.shape[0] < B:
         raise ValueError("block table has fewer rows than the batch")
